@@ -4,6 +4,7 @@
 #include "hp_core.h"
 #include "hp_cosmo.h"
 #include "hp_kernels.h"
+#include "hp_reduce.h"
 
 namespace hp {
 
@@ -37,26 +38,27 @@ __global__ void __launch_bounds__(256) fill_axis(double* f0, double* f1, double*
     f0[qd] = f0[qs]; f1[qd] = f1[qs]; f2[qd] = f2[qs]; f3[qd] = f3[qs]; f4[qd] = f4[qs];
 }
 
-// CFL maximum over the interior, hydropad/speed.F90:22-31.
+// CFL maximum over the interior, hydropad/speed.F90:22-31.  Bound by HBM
+// (40 B per cell); indices are 32-bit (a box has fewer than 2^31 cells), as
+// 64-bit divisions would cost more than the loads.
 __global__ void __launch_bounds__(256) speed_kernel(const double* __restrict__ p, const double* __restrict__ rho,
                                                     const double* __restrict__ vx, const double* __restrict__ vy,
                                                     const double* __restrict__ vz, int nx, int ny, int nz, int nb,
                                                     const Params* __restrict__ prm, DevStatus* st)
 {
-    const int Nx = nx - 2 * nb, Ny = ny - 2 * nb, Nz = nz - 2 * nb;
-    const long tot = (long)Nx * Ny * Nz;
+    const unsigned Nx = nx - 2 * nb, Ny = ny - 2 * nb, Nz = nz - 2 * nb;
+    const unsigned tot = Nx * Ny * Nz;
     const double gamma = prm->gamma;
     double vmax = 0.0;
-    for (long t = (long)blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += (long)gridDim.x * blockDim.x) {
-        const long i = t % Nx, r = t / Nx;
-        const long j = r % Ny, k = r / Ny;
+    for (unsigned t = blockIdx.x * blockDim.x + threadIdx.x; t < tot; t += gridDim.x * blockDim.x) {
+        const unsigned r = t / Nx, i = t - r * Nx;
+        const unsigned k = r / Ny, j = r - k * Ny;
         const long q = (nb + i) + (long)nx * ((nb + j) + (long)ny * (nb + k));
         const double vs = sqrt(gamma * p[q] / rho[q]);
         vmax = tmax(vmax, tmax(tmax(fabs(vx[q]), fabs(vy[q])), fabs(vz[q])) + vs);
     }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) vmax = fmax(vmax, __shfl_xor(vmax, off, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(&st->velmax_bits, (unsigned long long)__double_as_longlong(vmax));
+    const unsigned long long bits = block_max_bits(vmax);
+    if (threadIdx.x == 0) raise_velmax(st, bits);
 }
 
 // timedet, hydropad/functions.F90:2-35 (non-cosmological branch).

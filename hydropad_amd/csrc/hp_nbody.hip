@@ -16,6 +16,7 @@
 
 #include "hp_core.h"
 #include "hp_kernels.h"
+#include "hp_reduce.h"
 
 namespace hp {
 
@@ -85,13 +86,11 @@ __device__ __forceinline__ void drift1(double rdtath, const double bs[3], double
 __device__ __forceinline__ void flush_particles(DevStatus* st, unsigned long long outside, double vmax, bool speed)
 {
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        outside += __shfl_xor(outside, off, 64);
-        if (speed) vmax = fmax(vmax, __shfl_xor(vmax, off, 64));
-    }
-    if ((threadIdx.x & 63) == 0) {
-        if (outside) atomicAdd(&st->outside, outside);
-        if (speed) atomicMax(&st->velmax_bits, (unsigned long long)__double_as_longlong(vmax));
+    for (int off = 32; off >= 1; off >>= 1) outside += __shfl_xor(outside, off, 64);
+    if ((threadIdx.x & 63) == 0 && outside) atomicAdd(&st->outside, outside);
+    if (speed) {                                         // the same for every thread of the launch
+        const unsigned long long bits = block_max_bits(vmax);
+        if (threadIdx.x == 0) raise_velmax(st, bits);
     }
 }
 

@@ -23,6 +23,7 @@
 #include "hp_core.h"
 #include "hp_fast.h"
 #include "hp_kernels.h"
+#include "hp_reduce.h"
 
 namespace hp {
 
@@ -345,7 +346,19 @@ __device__ __forceinline__ void finish_cell(const BoxView& B, const Epilogue& E,
     store_cell(B.out, q, val, ix, iy, iz, E.ghost_mask, B.nx, B.ny, B.nz, B.nb);
 }
 
-// Wave-level reduction of the per-lane counters, then one atomic per wave.
+// The atomics of one wave's or block's tallies (hp_reduce.h); most have
+// nothing to raise.
+__device__ __forceinline__ void raise_counters(DevStatus* st, int nitmax, int nonconv, int nclamp, double vmax,
+                                               bool want_speed)
+{
+    if (nitmax > __hip_atomic_load(&st->newton_max, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+        atomicMax(&st->newton_max, nitmax);
+    if (nonconv) atomicAdd(&st->newton_nonconv, (unsigned long long)nonconv);
+    if (nclamp) atomicAdd(&st->clamps, (unsigned long long)nclamp);
+    if (want_speed) raise_velmax(st, (unsigned long long)__double_as_longlong(vmax));
+}
+
+// Wave-level reduction of the per-lane counters, then one wave's atomics.
 __device__ __forceinline__ void flush_counters(DevStatus* st, const Tally& T, bool want_speed)
 {
     int nitmax = T.nitmax, nonconv = T.nonconv, nclamp = T.nclamp;
@@ -357,12 +370,7 @@ __device__ __forceinline__ void flush_counters(DevStatus* st, const Tally& T, bo
         nclamp += __shfl_xor(nclamp, off, 64);
         if (want_speed) vmax = fmax(vmax, __shfl_xor(vmax, off, 64));
     }
-    if ((threadIdx.x & 63) == 0) {
-        if (nitmax > 0) atomicMax(&st->newton_max, nitmax);
-        if (nonconv) atomicAdd(&st->newton_nonconv, (unsigned long long)nonconv);
-        if (nclamp) atomicAdd(&st->clamps, (unsigned long long)nclamp);
-        if (want_speed) atomicMax(&st->velmax_bits, (unsigned long long)__double_as_longlong(vmax));
-    }
+    if ((threadIdx.x & 63) == 0) raise_counters(st, nitmax, nonconv, nclamp, vmax, want_speed);
 }
 
 // Block-level form for the single-box kernels: the waves' partial results
@@ -398,10 +406,7 @@ __device__ __forceinline__ void flush_counters_block(DevStatus* st, const Tally&
             nclamp += s_cl[k];
             vmax = fmax(vmax, s_vm[k]);
         }
-        if (nitmax > 0) atomicMax(&st->newton_max, nitmax);
-        if (nonconv) atomicAdd(&st->newton_nonconv, (unsigned long long)nonconv);
-        if (nclamp) atomicAdd(&st->clamps, (unsigned long long)nclamp);
-        if (want_speed) atomicMax(&st->velmax_bits, (unsigned long long)__double_as_longlong(vmax));
+        raise_counters(st, nitmax, nonconv, nclamp, vmax, want_speed);
     }
 }
 
