@@ -59,8 +59,8 @@ struct SweepLaunch {
     int dir;          // 1,2,3
     int ghost_mask;   // bit d-1: also write the periodic face-ghost images along axis d
     int do_speed;     // fuse the CFL maximum into this sweep
-    int seglen;       // streaming segment length for y/z sweeps (<= 0: whole pencil)
-    int xcpw;         // x sweep: chunks per wave (<= 0: about 16 resident rounds)
+    int seglen;       // streaming segment length for y/z sweeps (<= 0: stream_seglen)
+    int xcpw;         // x sweep: chunks per wave (<= 0: 16, fewer for small boxes)
     int block;        // threads per block
     int precision;    // Precision
     bool grav, cosmo;
@@ -71,6 +71,37 @@ struct SweepLaunch {
     const double* old[4];
     const double* fac;
 };
+
+// Waves of the y/z sweeps the chip holds at once: 256 CUs x 4 SIMDs, two
+// waves per SIMD for the gamma = 5/3 and the mixed kernels, one for the
+// others (256 registers and more).
+constexpr int STREAM_SLOTS = 1024;
+
+// Segment length of a y/z sweep whose pencils are `nax` cells long and take
+// `waves(nseg)` waves when each is split into nseg segments.  A wave walks a
+// segment of len cells in len + 6 iterations, the first four of them cheap:
+// about len + 4 cells' time, and the waves run in rounds of `slots`.  The
+// split with the smallest rounds x (len + 4) is taken, at most 64 cells long
+// (longer ones gain nothing on large boxes: 256^3 comoving 1265 us at 64 and
+// 1286 at 128, and leave fewer waves to even out the Newton iterations).
+// Measured, y sweep in us, one split near 64 cells against the one taken:
+// 32^3 tube 84 -> 17 (len 1), 64^3 tube 158 -> 26 (len 2), 96^3 comoving 468
+// -> 97 (len 7: 2016 waves), 128^3 455 -> 184 (len 16: 2048), 192^3 671 ->
+// 570 (len 28: 4032 waves, two rounds); just past a full round it is slower
+// (96^3 at len 6, 2304 waves: 127).
+template <class Waves> inline int stream_seglen(int nax, int slots, Waves waves)
+{
+    int best = nax < 64 ? nax : 64;
+    long cost = -1;
+    for (int nseg = (nax + best - 1) / best; nseg <= nax; ++nseg) {
+        const int len = (nax + nseg - 1) / nseg;
+        const long rounds = (waves((nax + len - 1) / len) + slots - 1) / slots;
+        const long c = rounds * (len + 4);
+        if (cost < 0 || c < cost) { cost = c; best = len; }
+        if (rounds * 5 > cost) break;                  // shorter segments only cost more from here
+    }
+    return best;
+}
 
 hipError_t launch_sweep(const BoxView& b, const SweepLaunch& L, hipStream_t s);
 // Periodic ghost fill of the 5 fields of `f` (in place); dir 1..3 or 0 = all (z, x, y).

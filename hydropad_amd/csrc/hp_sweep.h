@@ -692,12 +692,17 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
             Face<double> fL = fRprev, fR = fRprev;
             const int ic = kk - 2;                                   // cell k-2, interface at its left
             if (kk >= s0 + 1) {     // parabola and faces of cell k-2
-                // clamp count: both faces of the cells s0-1 .. s1 a segment
-                // reconstructs (per interface only in the x sweep: an exact
-                // count here costs the FP64 form half its occupancy)
+                int nclL = 0, nclR = 0;
                 const bool flat = flat_always || bits != 0u || bk;
                 M::template cell_faces<R, NV, GRAV, COSMO>(A, w2, iv2, iv1, w0[VR], w1[VR], w3[VR], cur[VR], d1[VR],
-                                                           d3[VR], w1[VP], w3[VP], flat, fL, fR, T.nclamp, T.nclamp);
+                                                           d3[VR], w1[VP], w3[VP], flat, fL, fR, nclL, nclR);
+                // clamps once per interface of the pencil (0 .. Nax), as the
+                // reference's loop counts them: a segment takes those of its
+                // own cells, the pencil's ends one face beyond
+                if (nclL + nclR) {
+                    if (kk - 2 >= s0 && (kk - 2 < s1 || s1 == Nax)) T.nclamp += nclL;
+                    if ((kk - 2 >= s0 || s0 == 0) && kk - 2 < s1) T.nclamp += nclR;
+                }
             }
             Flux F = Fprev;
             if (kk >= s0 + 2) {     // Riemann problem at interface k-2
@@ -773,8 +778,6 @@ static hipError_t launch_sweep_t(const BoxView& b, const SweepLaunch& L, hipStre
     if (L.dir == 1) {
         const long total = (long)Ny * Nz * b.nx;
         const long nchunks = (total + 57) / 58;
-        // about 16 resident rounds of waves over 256 CUs x 4 SIMDs; each wave
-        // walks its run of chunks with a one-chunk register prefetch
         // waves of 16 chunks (fewer for small boxes, to keep ~16K waves):
         // short runs balance the divergent Riemann work across the chip
         long cpw = std::min<long>(16, nchunks / 16384);
@@ -787,12 +790,11 @@ static hipError_t launch_sweep_t(const BoxView& b, const SweepLaunch& L, hipStre
     } else {
         const int Nax = (L.dir == 2) ? Ny : Nz;
         const int Nbb = (L.dir == 2) ? Nz : Ny;
-        // default: split pencils into segments of at least 64 cells until there
-        // are ~16K waves (each segment recomputes a 6-cell halo)
         int seglen = L.seglen;
         if (seglen <= 0) {
-            const long npen = (long)Nx * ((L.dir == 2) ? Nz : Ny);
-            seglen = (int)std::min<long>(Nax, std::max<long>(64, (long)Nax * npen / (16384L * 64)));
+            const long npen = (long)Nx * Nbb;
+            const int slots = STREAM_SLOTS * (M::G53 || sizeof(R) == 4 ? 2 : 1);
+            seglen = stream_seglen(Nax, slots, [&](int nseg) { return (npen * nseg + 63) / 64; });
         }
         if (seglen > Nax) seglen = Nax;
         const int nseg = (Nax + seglen - 1) / seglen;

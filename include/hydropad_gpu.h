@@ -177,9 +177,9 @@ int hp_expand(hp_ctx* ctx, double afact);
 int hp_evolve_cosmo(hp_ctx* ctx, int first_step, int nsteps, hp_cosmo* s);
 
 /* Launch shape of this context's sweeps: x_chunks = 58-cell chunks each
- * x-sweep wave walks (0: about 16 resident rounds of waves), yz_seglen =
- * y/z pencil segment length (0: at least 64 cells, short enough for ~16K
- * waves), block = threads per block
+ * x-sweep wave walks (0: 16, fewer for small boxes), yz_seglen =
+ * y/z pencil segment length (0: at most 64 cells, shorter where the box
+ * would not fill the GPU), block = threads per block
  * (0: 256; a multiple of 64, at most 256).  The shape never changes a result.
  * No reference counterpart (the reference's OpenACC gang/vector shapes are
  * compiler-chosen). */
@@ -246,7 +246,8 @@ typedef struct hp_batch hp_batch;
 
 typedef struct hp_batch_tuning {
     int x_chunks;         /* x sweep: 58-cell chunks per work unit (0: 4) */
-    int yz_segments;      /* y/z sweeps: segments each pencil is split into (0: 1) */
+    int yz_segments;      /* y/z sweeps: segments each pencil is split into (0: as many as the boxes
+                             present need to fill the GPU) */
     int waves_per_cu;     /* persistent grid: waves per compute unit (0: 8) */
     int reserved;
 } hp_batch_tuning;

@@ -8,6 +8,7 @@ import pytest
 import hydropad_amd as hp
 from helpers import FIELDS, NB, copy_state, rel_l1, to_hp_params
 from hydropad_amd import ic
+from oracle import HpCounters as OracleCounters
 
 pytestmark = pytest.mark.gpu
 
@@ -94,3 +95,33 @@ def test_sweeps_write_the_periodic_face_ghosts(precision, shape):
                     hi_g[ax], hi_src[ax] = slice(n + NB, n + 2 * NB), slice(NB, 2 * NB)
                     assert np.array_equal(a[tuple(lo_g)], a[tuple(lo_src)]), (precision, shape, d, tiling, k, ax, "low")
                     assert np.array_equal(a[tuple(hi_g)], a[tuple(hi_src)]), (precision, shape, d, tiling, k, ax, "high")
+
+
+@pytest.mark.parametrize("shape", [(3, 3, 3), (16, 16, 16), (40, 33, 29), (9, 130, 66), (130, 67, 9)],
+                         ids=lambda s: "x".join(map(str, s)))
+def test_default_segments_match_whole_pencils(oracle, shape):
+    """The y/z segment length the launch chooses (from one cell for the
+    smallest boxes to 64) against whole pencils and lengths around it: the
+    same bits, and the same Newton and clamp counts as the oracle's, which
+    count each interface once.  Courant number 4 makes some traced states
+    negative in the noisy box, so there is something to count."""
+    st = random_box(shape, 7 + shape[1], amp=3.0, vamp=2.0)
+    P = oracle.params(ngrid=max(shape))
+    oracle.timedet(P, oracle.speed(P, st), 4.0, 1e30, 0.0)
+    for d in (2, 3):
+        cnt = OracleCounters()
+        oracle.ppmsolver(P, copy_state(st), d, counters=cnt)
+        base = None
+        for seglen in (0, 1, 2, 7, 64, 4096):
+            with hp.Box(st["p"].shape, "fp64") as box:
+                box.set_params(to_hp_params(P, hp.HpParams))
+                box.set_tiling(0, seglen, 0)
+                box.upload(copy_state(st))
+                box.reset_counters()
+                box.ppmsolver(d)
+                c, out = box.counters(), box.download()
+            assert c.neg_state_clamps == cnt.neg_state_clamps, (shape, d, seglen)
+            base = base or (out, c.newton_iters_max)
+            assert c.newton_iters_max == base[1], (shape, d, seglen)
+            for k in FIELDS:
+                assert np.array_equal(out[k], base[0][k]), (shape, d, seglen, k)
