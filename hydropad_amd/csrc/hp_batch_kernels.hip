@@ -111,7 +111,7 @@ __global__ void __launch_bounds__(256) batch_x(const BatchBox* __restrict__ boxe
 // with no spill.  (The general-gamma FP64 bodies need ~290; forced to two
 // waves they spill about 1 KB per lane, so they are left to the allocator.)
 template <class M, class R, int DIR, bool EXP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((M::G53 || sizeof(R) == 4) ? 2 : 1)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, false>())))
 batch_stream(const BatchBox* __restrict__ boxes, const BatchPlan* __restrict__ plan, int key, int slot)
 {
     const BatchTable& T = plan->t[key];

@@ -743,8 +743,18 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
     }
 }
 
+// Waves per SIMD a y/z kernel is built for.  Two for gamma = 5/3 and the mixed
+// forms, held there where the allocator would take a register or two over the
+// 256 they allow (gamma = 5/3 FP64 with gravity); the general-gamma FP64
+// forms, and its mixed one with gravity, would spill and keep one.
+template <class M, class R, bool GRAV> constexpr int stream_waves()
+{
+    return (M::G53 || (sizeof(R) == 4 && !GRAV)) ? 2 : 1;
+}
+
 template <class M, class R, int DIR, bool GRAV, bool COSMO, bool EXP>
-__global__ void __launch_bounds__(256) sweep_stream(BoxView B, Epilogue E, int seglen, int nseg)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, GRAV>())))
+sweep_stream(BoxView B, Epilogue E, int seglen, int nseg)
 {
     if (EXP) load_factors(E);
     int Nax, Nbb;
@@ -793,7 +803,7 @@ static hipError_t launch_sweep_t(const BoxView& b, const SweepLaunch& L, hipStre
         int seglen = L.seglen;
         if (seglen <= 0) {
             const long npen = (long)Nx * Nbb;
-            const int slots = STREAM_SLOTS * (M::G53 || sizeof(R) == 4 ? 2 : 1);
+            const int slots = STREAM_SLOTS * stream_waves<M, R, G>();
             seglen = stream_seglen(Nax, slots, [&](int nseg) { return (npen * nseg + 63) / 64; });
         }
         if (seglen > Nax) seglen = Nax;
