@@ -72,8 +72,10 @@ __host__ __device__ inline int batch_current(int nsets, long long n)
     return nsets == 2 ? (int)(n & 1) : (int)(n % 3);
 }
 
+// grid: blocks at most; no more are launched than ncu CUs hold at once, as the
+// units are dealt out over the grid.
 hipError_t launch_batch_sweep(const BatchBox* boxes, const BatchPlan* plan, int slot, int dir, int prec, int exp,
-                              int g53, int grid, hipStream_t s);
+                              int g53, int grid, int ncu, hipStream_t s);
 
 }  // namespace hp
 

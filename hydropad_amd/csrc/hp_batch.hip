@@ -175,9 +175,11 @@ size_t field_bytes(int nx, int ny, int nz)
     return ((size_t)nx * ny * nz * sizeof(double) + align - 1) / align * align;
 }
 
+// Blocks of the persistent grid at the tuning's waves per CU; a kernel that
+// holds fewer at once takes those (launch_batch_sweep).
 int persistent_grid(const hp_batch* b)
 {
-    const int wpc = b->tune.waves_per_cu > 0 ? b->tune.waves_per_cu : 8;
+    const int wpc = b->tune.waves_per_cu > 0 ? b->tune.waves_per_cu : 16;
     return std::max(1, b->ncu * wpc / 4);
 }
 
@@ -199,8 +201,7 @@ void set_units(hp::BatchBox& X, const hp_batch_tuning& t, int len)
         const int nseg = (Nax + seglen - 1) / seglen;
         X.seglen[d] = seglen;
         X.nseg[d] = nseg;
-        const long items = (long)Nx * Nbb * nseg;
-        X.units[d + 1] = (int)((items + 63) / 64);
+        X.units[d + 1] = (int)hp::stream_items((long)Nx * Nbb, nseg);
     }
 }
 
@@ -229,19 +230,17 @@ int push_box(hp_batch* b, int id)
 // 57.5 ms with whole pencils, 30.1 ms with this rule.
 int tile_boxes(hp_batch* b)
 {
-    int nax = 1, slots = hp::STREAM_SLOTS;
+    int nax = 1;
     for (const hp::BatchBox& X : b->h_boxes)
-        if (X.active) {
-            nax = std::max(nax, std::max(X.ny, X.nz) - 2 * X.nb);
-            if (X.g53 || X.prec == hp::PREC_MIXED) slots = 2 * hp::STREAM_SLOTS;
-        }
+        if (X.active) nax = std::max(nax, std::max(X.ny, X.nz) - 2 * X.nb);
+    const int slots = 4 * std::min(persistent_grid(b), 3 * b->ncu);   // waves of a y/z sweep's grid
     const int len = hp::stream_seglen(nax, slots, [&](int nseg) {
         const int l = (nax + nseg - 1) / nseg;
         long waves = 0;
         for (const hp::BatchBox& X : b->h_boxes)
             if (X.active) {
                 const long Nx = X.nx - 2 * X.nb, Ny = X.ny - 2 * X.nb, Nz = X.nz - 2 * X.nb;
-                waves += (Nx * Ny * ((Nz + l - 1) / l) + 63) / 64;
+                waves += hp::stream_items(Nx * Ny, (int)((Nz + l - 1) / l));
             }
         return waves;
     });
@@ -277,11 +276,11 @@ int enqueue_step(hp_batch* b, unsigned combos, int grid)
                 if (!stat && !como) continue;
                 for (int dir = 1; dir <= 3; ++dir) {
                     if (slot < 2 || stat)
-                        if (hp::launch_batch_sweep(b->d_boxes, b->d_plan, slot, dir, prec, 0, g, grid, b->stream) !=
+                        if (hp::launch_batch_sweep(b->d_boxes, b->d_plan, slot, dir, prec, 0, g, grid, b->ncu, b->stream) !=
                             hipSuccess)
                             return HP_E_HIP;
                     if (slot == 2 && como)
-                        if (hp::launch_batch_sweep(b->d_boxes, b->d_plan, slot, dir, prec, 1, g, grid, b->stream) !=
+                        if (hp::launch_batch_sweep(b->d_boxes, b->d_plan, slot, dir, prec, 1, g, grid, b->ncu, b->stream) !=
                             hipSuccess)
                             return HP_E_HIP;
                 }
@@ -696,7 +695,7 @@ int hp_batch_autotune(hp_batch* b, int steps_per_trial, hp_batch_tuning* best, d
     if (graph_was) hp_batch_use_graph(b, 0);  // host-side capture time stays out of the timings
     hp_batch_tuning cur = b->tune;
     if (cur.x_chunks == 0) cur.x_chunks = 4;
-    if (cur.waves_per_cu == 0) cur.waves_per_cu = 8;
+    if (cur.waves_per_cu == 0) cur.waves_per_cu = 16;
     hipEvent_t e0, e1;
     HPCHK(hipEventCreate(&e0));
     HPCHK(hipEventCreate(&e1));

@@ -21,22 +21,6 @@ __device__ __forceinline__ int table_find(const BatchTable& T, int u)
     return lo;
 }
 
-// v with every 32-bit word taken from the wave's first active lane.  The
-// per-box descriptors and scalars are wave-uniform, but the kernel reads them
-// after its own counter atomics, through pointers it also writes, so the
-// compiler loads them per lane; this returns them to scalar registers.
-template <class T> __device__ __forceinline__ T wave_uniform(const T& v)
-{
-    static_assert(sizeof(T) % 4 == 0, "whole words");
-    int w[sizeof(T) / 4];
-    __builtin_memcpy(w, &v, sizeof(T));
-#pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 4; ++i) w[i] = __builtin_amdgcn_readfirstlane(w[i]);
-    T r;
-    __builtin_memcpy(&r, w, sizeof(T));
-    return r;
-}
-
 __device__ __forceinline__ void batch_view(const BatchBox& X, int slot, BoxView& V, Epilogue& E)
 {
     int in, out, old;
@@ -91,7 +75,7 @@ __global__ void __launch_bounds__(256) batch_x(const BatchBox* __restrict__ boxe
             cur = b;
         }
         const BatchBox& X = boxes[b];
-        const int local = u - T.start[i];
+        const int local = __builtin_amdgcn_readfirstlane(u - T.start[i]);
         BoxView V;
         Epilogue E;
         batch_view(X, slot, V, E);
@@ -111,49 +95,56 @@ __global__ void __launch_bounds__(256) batch_x(const BatchBox* __restrict__ boxe
 // with no spill.  (The general-gamma FP64 bodies need ~290; forced to two
 // waves they spill about 1 KB per lane, so they are left to the allocator.)
 template <class M, class R, int DIR, bool EXP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, false>())))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, false, true>())))
 batch_stream(const BatchBox* __restrict__ boxes, const BatchPlan* __restrict__ plan, int key, int slot)
 {
+    __shared__ double window[stream_lds<false>() * STREAM_BLOCK];
     const BatchTable& T = plan->t[key];
     const int total = T.total;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
-    const int lane = threadIdx.x & 63;
     // unit indices are wave-uniform; readfirstlane lets the table search and
     // the descriptor loads run on the scalar unit
     const int u0 = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     int cur = -1;
     Tally t = tally0();
+    double* const column = window + threadIdx.x;
+    reset_rare<false>(column);
     for (int u = u0; u < total; u += nwaves) {
         const int i = __builtin_amdgcn_readfirstlane(table_find(T, u));
         const int b = __builtin_amdgcn_readfirstlane(T.box[i]);
         if (b != cur) {
-            if (cur >= 0) flush_counters(boxes[cur].st, t, slot == 2);
+            if (cur >= 0) {
+                take_rare<false>(column, t);
+                flush_counters(boxes[cur].st, t, slot == 2);
+            }
             t = tally0();
+            reset_rare<false>(column);
             cur = b;
         }
         const BatchBox& X = boxes[b];
-        const int local = u - T.start[i];
+        const int local = __builtin_amdgcn_readfirstlane(u - T.start[i]);
         BoxView V;
         Epilogue E;
         batch_view(X, slot, V, E);
         const int Nbb = (DIR == 2) ? X.nz - 2 * X.nb : X.ny - 2 * X.nb;
-        const long npen = (long)(X.nx - 2 * X.nb) * Nbb;
-        const int nseg = X.nseg[DIR - 2];
-        const unsigned item = (unsigned)local * 64u + (unsigned)lane;   // items per box < 2^31
-        const bool active = (long)item < npen * nseg;
-        const unsigned it = active ? item : 0u;
-        const int seg = (int)(it / (unsigned)npen);
-        const long pen = (long)(it - (unsigned)seg * (unsigned)npen);
+        unsigned pen, seg;
+        const bool active = stream_item((unsigned)local, (unsigned)((X.nx - 2 * X.nb) * Nbb), pen, seg);
         const AllScalars<R> A = wave_uniform(load_scalars<M, R>(X.prm, X.st));
-        stream_run<M, R, DIR, false, true, EXP>(V, A, E, pen, seg, X.seglen[DIR - 2], active, t);
+        stream_run<M, R, DIR, false, true, EXP>(V, A, E, pen, (int)seg, X.seglen[DIR - 2], active, t, column);
     }
-    if (cur >= 0) flush_counters(boxes[cur].st, t, slot == 2);
+    if (cur >= 0) {
+        take_rare<false>(column, t);
+        flush_counters(boxes[cur].st, t, slot == 2);
+    }
 }
 
 template <class M, class R, bool EXP>
-static void launch_dir(const BatchBox* boxes, const BatchPlan* plan, int key, int slot, int dir, int grid,
-                       hipStream_t s)
+static void launch_dir(const BatchBox* boxes, const BatchPlan* plan, int key, int slot, int dir, int most,
+                       int ncu, hipStream_t s)
 {
+    // blocks of four waves a CU holds: one for each wave of a SIMD
+    constexpr int X = sizeof(R) == 4 ? (M::G53 ? 4 : 3) : (M::G53 ? 3 : 2);
+    const int grid = std::min(most, ncu * (dir == 1 ? X : stream_waves<M, R, false, true>()));
     if (dir == 1) hipLaunchKernelGGL((batch_x<M, R, EXP>), dim3(grid), dim3(256), 0, s, boxes, plan, key, slot);
     else if (dir == 2)
         hipLaunchKernelGGL((batch_stream<M, R, 2, EXP>), dim3(grid), dim3(256), 0, s, boxes, plan, key, slot);
@@ -162,24 +153,24 @@ static void launch_dir(const BatchBox* boxes, const BatchPlan* plan, int key, in
 
 template <class M>
 static void launch_m(const BatchBox* boxes, const BatchPlan* plan, int key, int slot, int dir, int prec, int exp,
-                     int grid, hipStream_t s)
+                     int grid, int ncu, hipStream_t s)
 {
     if (prec == PREC_MIXED) {
-        if (exp) launch_dir<M, float, true>(boxes, plan, key, slot, dir, grid, s);
-        else launch_dir<M, float, false>(boxes, plan, key, slot, dir, grid, s);
+        if (exp) launch_dir<M, float, true>(boxes, plan, key, slot, dir, grid, ncu, s);
+        else launch_dir<M, float, false>(boxes, plan, key, slot, dir, grid, ncu, s);
     } else {
-        if (exp) launch_dir<M, double, true>(boxes, plan, key, slot, dir, grid, s);
-        else launch_dir<M, double, false>(boxes, plan, key, slot, dir, grid, s);
+        if (exp) launch_dir<M, double, true>(boxes, plan, key, slot, dir, grid, ncu, s);
+        else launch_dir<M, double, false>(boxes, plan, key, slot, dir, grid, ncu, s);
     }
 }
 
 hipError_t launch_batch_sweep(const BatchBox* boxes, const BatchPlan* plan, int slot, int dir, int prec, int exp,
-                              int g53, int grid, hipStream_t s)
+                              int g53, int grid, int ncu, hipStream_t s)
 {
     if (slot < 0 || slot > 2 || dir < 1 || dir > 3 || grid < 1) return hipErrorInvalidValue;
     const int key = table_key(slot, dir, prec, exp, g53);
-    if (g53) launch_m<FastMath53>(boxes, plan, key, slot, dir, prec, exp, grid, s);
-    else launch_m<FastMath>(boxes, plan, key, slot, dir, prec, exp, grid, s);
+    if (g53) launch_m<FastMath53>(boxes, plan, key, slot, dir, prec, exp, grid, ncu, s);
+    else launch_m<FastMath>(boxes, plan, key, slot, dir, prec, exp, grid, ncu, s);
     return hipGetLastError();
 }
 

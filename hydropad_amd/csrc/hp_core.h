@@ -50,7 +50,7 @@ enum { VP = 0, VR = 1, VU = 2, VV = 3, VW = 4, VG = 5 };
 // block and converted to the reconstruction precision R.
 template <class R> struct SweepScalars {
     R gamma, dt, rat, dx, rdx, dat, at, flatvalue, mingradflat;
-    R dtrat;   // dt*rat, used only by the fast forms
+    R ktrace;  // dt*rat/dx, used only by the fast forms
     R cdat2;   // 2*dat*rat*dt (expansion term of beta/beta0), used only by the fast forms
 };
 
@@ -465,6 +465,7 @@ __device__ __forceinline__ void peak_floor(const RScal& R, Flux& F, double rb1, 
 // (pm1+pm2)*0.5 as in hydro/ppm.F90:583 (undefined in integrate.F90).
 struct IScal {
     double rdtath, rdx, gamma, rgamma1, eta1, eta2;
+    double lam;   // rdtath*rdx, used only by the fast forms
 };
 
 // Dual-energy selection, integrate.F90:196-216: eintnew enters as the

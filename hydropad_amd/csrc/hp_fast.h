@@ -331,7 +331,7 @@ __device__ __forceinline__ Face<double> trace_face_d(const SweepScalars<R>& S, c
                                                      double cs, double gamma, int& nclamp)
 {
     const double um = a[VU] - cs, u0 = a[VU], up = a[VU] + cs;     // characteristic speeds (FP64 signs)
-    const R k = S.dtrat * S.rdx;
+    const R k = S.ktrace;
     R xt, x1, x2, x3;
     if (RIGHT) {
         x3 = (R)up * k;
@@ -868,7 +868,7 @@ __device__ __forceinline__ void integrate_cell(const IScal& S, const Flux& F1, c
                                                double& rho, double& vx, double& vy, double& vz, double etot,
                                                double ghalf, bool grav)
 {
-    const double lam = S.rdtath * S.rdx, gamma = S.gamma, rgamma1 = S.rgamma1;
+    const double lam = S.lam, gamma = S.gamma, rgamma1 = S.rgamma1;
     const double eint = pres * rgamma1;
     const double m1 = F1.r * F1.u, m2 = F2.r * F2.u;     // mass fluxes
     double rhonew = rho + lam * (m1 - m2);

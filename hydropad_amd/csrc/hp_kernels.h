@@ -72,26 +72,28 @@ struct SweepLaunch {
     const double* fac;
 };
 
-// Waves of the y/z sweeps the chip holds at once: 256 CUs x 4 SIMDs, two
-// waves per SIMD for the gamma = 5/3 and the mixed kernels, one for the
-// others (256 registers and more).
+// Waves of a y/z sweep the chip holds at once, for each wave its SIMD holds:
+// 256 CUs x 4 SIMDs.
 constexpr int STREAM_SLOTS = 1024;
 
 // Segment length of a y/z sweep whose pencils are `nax` cells long and take
 // `waves(nseg)` waves when each is split into nseg segments.  A wave walks a
 // segment of len cells in len + 6 iterations, the first four of them cheap:
 // about len + 4 cells' time, and the waves run in rounds of `slots`.  The
-// split with the smallest rounds x (len + 4) is taken, at most 64 cells long
-// (longer ones gain nothing on large boxes: 256^3 comoving 1265 us at 64 and
-// 1286 at 128, and leave fewer waves to even out the Newton iterations).
-// Measured, y sweep in us, one split near 64 cells against the one taken:
-// 32^3 tube 84 -> 17 (len 1), 64^3 tube 158 -> 26 (len 2), 96^3 comoving 468
-// -> 97 (len 7: 2016 waves), 128^3 455 -> 184 (len 16: 2048), 192^3 671 ->
-// 570 (len 28: 4032 waves, two rounds); just past a full round it is slower
-// (96^3 at len 6, 2304 waves: 127).
+// split with the smallest rounds x (len + 4) is taken, at most 24 cells long:
+// short enough that the waves that got the most Newton iterations do not run
+// on alone, and that the rows two segments share are still in cache.  Measured, y sweep in us, by length (taken one in brackets):
+//   64^3 tube                 64: 155   16: 49   8: 33   [2]: 24
+//   96^3 comoving             48: 353   16: 133  7: 94   [5]: 96   4: 107
+//   128^3 comoving            64: 448   32: 245  16: 174 [11]: 167  10: 181
+//   192^3 comoving            64: 640   28: 503  24: 520 [20]: 475  18: 491
+//   256^3 comoving            64: 1053  32: 1010 24: 984 [22]: 1042 16: 1023
+//   512^3 tube                128: 3270 64: 3132 32: 2995 [20]: 2854 16: 2811
+// A length just past a full round (10 at 128^3, 24 at 192^3) is slower than
+// its neighbours.
 template <class Waves> inline int stream_seglen(int nax, int slots, Waves waves)
 {
-    int best = nax < 64 ? nax : 64;
+    int best = nax < 24 ? nax : 24;
     long cost = -1;
     for (int nseg = (nax + best - 1) / best; nseg <= nax; ++nseg) {
         const int len = (nax + nseg - 1) / nseg;
@@ -102,6 +104,9 @@ template <class Waves> inline int stream_seglen(int nax, int slots, Waves waves)
     }
     return best;
 }
+
+// Waves of a y/z sweep of npen pencils in nseg segments each (hp_sweep.h).
+inline long stream_items(long npen, int nseg) { return (npen + 255) / 256 * 4 * nseg; }
 
 hipError_t launch_sweep(const BoxView& b, const SweepLaunch& L, hipStream_t s);
 // Periodic ghost fill of the 5 fields of `f` (in place); dir 1..3 or 0 = all (z, x, y).

@@ -126,6 +126,13 @@ __device__ __forceinline__ double total_phys(double rgamma1, double p, double r,
     return p * rgamma1 + 0.5 * r * (vx * vx + vy * vy + vz * vz);
 }
 
+// Element q of a field.  The pointers of a batch's boxes come from memory, so
+// without the address space the compiler would make flat accesses of them,
+// which count as LDS traffic too and make every LDS wait one for memory.
+typedef __attribute__((address_space(1))) double gdouble;
+__device__ __forceinline__ double at(const double* f, long q) { return ((const gdouble*)f)[q]; }
+__device__ __forceinline__ void put(double* f, long q, double v) { ((gdouble*)f)[q] = v; }
+
 // ---- DPP whole-wave shifts (gfx9 wave_shr:1 / wave_shl:1) -------------------
 constexpr int DPP_WAVE_SHL1 = 0x130;   // lane l receives lane l+1
 constexpr int DPP_WAVE_SHR1 = 0x138;   // lane l receives lane l-1
@@ -171,6 +178,26 @@ template <class R> struct AllScalars {
     double rgamma1, gamma, mingradflat;
 };
 
+// v with every 32-bit word taken from the wave's first active lane.  A box's
+// descriptor and scalars are wave-uniform, but what the vector unit derived
+// from them (there is no scalar FP64 arithmetic), or what a batch kernel reads
+// after its own counter atomics, through pointers it also writes, sits in
+// vector registers; this returns it to scalar ones.
+template <class T> __device__ __forceinline__ T wave_uniform(const T& v)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    int w[sizeof(T) / 4];
+    __builtin_memcpy(w, &v, sizeof(T));
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) {
+        if (!__builtin_constant_p(w[i])) asm("" : "+v"(w[i]));   // else a uniform value is left where it is
+        w[i] = __builtin_amdgcn_readfirstlane(w[i]);
+    }
+    T r;
+    __builtin_memcpy(&r, w, sizeof(T));
+    return r;
+}
+
 // gamma-derived constants for gamma = 5/3, by the expressions of
 // hydropad/initialize_parameters.F90:64-69 (and hp_params_init)
 struct Gamma53 {
@@ -200,7 +227,7 @@ __device__ __forceinline__ AllScalars<R> load_scalars(const Params* __restrict__
     A.S.gamma = (R)gamma; A.S.dt = (R)P.dt; A.S.rat = (R)P.rat; A.S.dx = (R)P.dx;
     A.S.rdx = (R)P.rdx; A.S.dat = (R)P.dat; A.S.at = (R)P.at;
     A.S.flatvalue = (R)P.flatvalue; A.S.mingradflat = (R)P.mingradflat;
-    A.S.dtrat = (R)(P.dt * P.rat);
+    A.S.ktrace = (R)(P.dt * P.rat) * A.S.rdx;
     A.S.cdat2 = (R)(2.0 * P.dat * P.rat * P.dt);
     A.Rs.gamma = gamma; A.Rs.gamma1 = gamma1; A.Rs.rgamma = rgamma; A.Rs.rgamma1 = rgamma1;
     A.Rs.m = m; A.Rs.rm = rm; A.Rs.gf = gf;
@@ -209,7 +236,7 @@ __device__ __forceinline__ AllScalars<R> load_scalars(const Params* __restrict__
     A.Rs.m5 = m5;
     A.Rs.nmax = cap > 0 ? cap : K_NNEWTMAX;
     A.Rs.nskip = K_NNEWTMAX - A.Rs.nmax;
-    A.Is.rdtath = P.rdtath; A.Is.rdx = P.rdx; A.Is.gamma = gamma; A.Is.rgamma1 = rgamma1;
+    A.Is.rdtath = P.rdtath; A.Is.rdx = P.rdx; A.Is.lam = P.rdtath * P.rdx; A.Is.gamma = gamma; A.Is.rgamma1 = rgamma1;
     A.Is.eta1 = P.eta1; A.Is.eta2 = P.eta2;
     A.rgamma1 = rgamma1; A.gamma = gamma; A.mingradflat = P.mingradflat;
     return A;
@@ -261,10 +288,10 @@ __device__ __forceinline__ void store_cell(double* const* out, long q, const dou
                                            int mask, int nx, int ny, int nz, int nb)
 {
 #pragma unroll
-    for (int f = 0; f < 5; ++f) out[f][q] = val[f];
+    for (int f = 0; f < 5; ++f) put(out[f], q, val[f]);
     auto image = [&](long shift) {
 #pragma unroll
-        for (int f = 0; f < 5; ++f) out[f][q + shift] = val[f];
+        for (int f = 0; f < 5; ++f) put(out[f], q + shift, val[f]);
     };
     if (mask & 1) {
         const int N = nx - 2 * nb;
@@ -317,9 +344,9 @@ __device__ __forceinline__ Tally tally0()
 // afact1 = 1/(1+afact), afact2 = 1/(2+afact) come precomputed (expand.F90:19-20).
 __device__ __forceinline__ void expand_cell(const Epilogue& E, long q, double* val)
 {
-    const double po = E.old[0][q];
+    const double po = at(E.old[0], q);
 #pragma unroll
-    for (int f = 2; f < 5; ++f) val[f] = (2.0 * val[f] - E.afact * E.old[f - 1][q]) * E.afact2;
+    for (int f = 2; f < 5; ++f) val[f] = (2.0 * val[f] - E.afact * at(E.old[f - 1], q)) * E.afact2;
     const double ppp = val[0];
     double pn = (val[0] - E.afact * po) * E.afact1;
     if (pn <= 0.0) pn = (ppp > 0.0) ? ppp : po;
@@ -451,9 +478,9 @@ __device__ __forceinline__ void x_run(const BoxView& B, const AllScalars<R>& A, 
         q = i + (long)nx * (j + (long)ny * k);
     };
     auto load = [&](long q, double* cd) {
-        cd[VP] = B.in[0][q]; cd[VR] = B.in[1][q];
-        cd[VU] = B.in[D::U][q]; cd[VV] = B.in[D::V][q]; cd[VW] = B.in[D::W][q];
-        if (GRAV) cd[NV - 1] = -B.gforce[3 * q + 0];
+        cd[VP] = at(B.in[0], q); cd[VR] = at(B.in[1], q);
+        cd[VU] = at(B.in[D::U], q); cd[VV] = at(B.in[D::V], q); cd[VW] = at(B.in[D::W], q);
+        if (GRAV) cd[NV - 1] = -at(B.gforce, 3 * q + 0);
     };
 
     // The FP64 form prefetches the next chunk into registers; the mixed form
@@ -601,9 +628,59 @@ template <int DIR> __device__ __forceinline__ void stream_geometry(const BoxView
     else { Nax = B.nz - 2 * nb; Nbb = B.ny - 2 * nb; s_ax = (long)B.nx * B.ny; s_b = B.nx; }
 }
 
+// The work of one of stream_items' waves: a lane per pencil, one segment for
+// all, so that the loop over the segment and its guards are scalar.  Four
+// consecutive waves take 256 consecutive pencils, whose rows are 2 KB of
+// memory, and a segment of all pencils comes before the next (one wave's 512
+// bytes at a time with the segments side by side: 512x512x256 tube 1405 ->
+// 1704 us, 256^3 comoving 1065 -> 1110).
+__device__ __forceinline__ bool stream_item(unsigned wave, unsigned npen, unsigned& pen, unsigned& seg)
+{
+    const unsigned groups = (npen + 255u) >> 8, four = wave >> 2;
+    seg = four / groups;
+    pen = ((four - seg * groups) * 4u + (wave & 3u)) * 64u + (threadIdx.x & 63u);
+    const bool active = pen < npen;
+    if (!active) pen = 0u;
+    return active;
+}
+
+// The window a thread slides along its segment lives in LDS, one column of
+// doubles per thread: a ring of the last four cells and the flux at the
+// interface behind.  Only the thread itself reads its column, so nothing
+// synchronises; consecutive lanes' columns are consecutive doubles.  Kept in
+// registers the window took the gamma = 5/3 kernels to 229 of them and two
+// waves per SIMD, and the VALU was busy 71 % of the time (the x sweep's three
+// waves: 92 %); a third wave fits beside the window in LDS.  Measured, y sweep
+// in us with its segment length, before and after: 256^3 comoving FP64 1194 ->
+// 1042, mixed 1068 -> 907, 160^3 gamma 1.66666667 (one wave -> two) 656 -> 494;
+// the 512^3 tube is bound by HBM (10.7 GB, 3.8 TB/s) and stays (2782 -> 2850).
+constexpr int STREAM_BLOCK = 256;                      // threads per block at most
+template <bool GRAV> constexpr int stream_window() { return 4 * (GRAV ? 6 : 5) + 5; }
+template <bool GRAV> constexpr int stream_lds() { return stream_window<GRAV>() + 1; }
+
+// The tallies that hardly ever change, clamps and iterations that did not
+// converge, are the two words of the column's last double.
+template <bool GRAV> __device__ __forceinline__ int* rare_tallies(double* column)
+{
+    return (int*)(column + stream_window<GRAV>() * STREAM_BLOCK);
+}
+
+template <bool GRAV> __device__ __forceinline__ void reset_rare(double* column)
+{
+    int* const rare = rare_tallies<GRAV>(column);
+    rare[0] = rare[1] = 0;
+}
+
+template <bool GRAV> __device__ __forceinline__ void take_rare(double* column, Tally& T)
+{
+    const int* const rare = rare_tallies<GRAV>(column);
+    T.nclamp = rare[0];
+    T.nonconv = rare[1];
+}
+
 template <class M, class R, int DIR, bool GRAV, bool COSMO, bool EXP>
-__device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>& A, const Epilogue& E, long pen,
-                                           int seg, int seglen, bool active, Tally& T)
+__device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>& A, const Epilogue& E, unsigned pen,
+                                           int seg, int seglen, bool active, Tally& T, double* column)
 {
     using D = Dirmap<DIR>;
     constexpr int NV = GRAV ? 6 : 5;
@@ -612,65 +689,68 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
     int Nax, Nbb;
     long s_ax, s_b;
     stream_geometry<DIR>(B, Nax, Nbb, s_ax, s_b);
-    const unsigned upen = (unsigned)pen;                 // pencils per box < 2^31
-    const int ib = (int)(upen / (unsigned)Nx), ia = (int)(upen - (unsigned)ib * (unsigned)Nx);
+    const int ib = (int)(pen / (unsigned)Nx), ia = (int)(pen - (unsigned)ib * (unsigned)Nx);
     const int s0 = seg * seglen;
     const int s1 = min(s0 + seglen, Nax);
     const long base = (nb + ia) + (long)(nb + ib) * s_b + (long)nb * s_ax;   // interior cell 0 of the pencil
     const bool flat_always = A.mingradflat <= 0.0;
 
-    double w0[NV], w1[NV], w2[NV], w3[NV];   // cells k-4 .. k-1
-    double r5 = 0.0;                         // rho of cell k-5
-    R d1[NV], d2[NV];                        // slopes of cells k-3, k-2
+    auto cell = [&](int it) { return column + (it & 3) * NV * STREAM_BLOCK; };   // cell loaded in iteration `it`
+    double* const flux = column + 4 * NV * STREAM_BLOCK;                          // flux at interface k-3
+    int* const rare = rare_tallies<GRAV>(column);
+    double w0r = 0.0;                        // rho of cell k-4
+    R d1r = R(0), d2[NV];                    // slopes of cells k-3 (rho), k-2
     double iv2[NV];                          // interface value at k-2 (left of cell k-2)
     unsigned bits = 0;                       // pair bits of k-3, k-2, k-1
     Face<double> fRprev;                     // right face of cell k-3
-    Flux Fprev;                              // flux at interface k-3 (left of cell k-3)
 #pragma unroll
-    for (int s = 0; s < NV; ++s) { w0[s] = w1[s] = w2[s] = w3[s] = iv2[s] = 0.0; d1[s] = d2[s] = R(0); }
+    for (int s = 0; s < NV; ++s) { iv2[s] = 0.0; d2[s] = R(0); }
     fRprev.p = fRprev.r = fRprev.u = fRprev.v = fRprev.w = 0.0;
-    Fprev.p = Fprev.r = Fprev.u = Fprev.v = Fprev.w = 0.0;
 
-    // The stores of the cell updated in one iteration are issued at the top of
-    // the next, before that iteration's prefetch: the wait for the prefetched
-    // values (vmcnt counts stores as well as loads) then finds both a whole
-    // iteration old instead of stalling on stores issued just before it.  The
-    // comoving kernels keep the store in place (the five values held across
-    // the iteration boundary would cost them occupancy or spills) and take
-    // delivery of the prefetch before it instead.
-    constexpr bool DEFER = !COSMO;
-    double pend[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     const int ixc = nb + ia, ibc = nb + ib;
-    auto store_pending = [&](int kc) {                 // cell kc of the segment, updated last iteration
-        const int ic = nb + kc;
-        if (DIR == 2) store_cell(B.out, base + (long)kc * s_ax, pend, ixc, ic, ibc, E.ghost_mask, B.nx, B.ny, B.nz, nb);
-        else store_cell(B.out, base + (long)kc * s_ax, pend, ixc, ibc, ic, E.ghost_mask, B.nx, B.ny, B.nz, nb);
-    };
+
+    // The next cell's loads go out at the top of an iteration and are taken
+    // delivery of before its stores; in the FP64 comoving kernels, whose
+    // tracing and Riemann phases leave no registers to hold them, they go out
+    // after those and arrive at the next head.
+    constexpr bool EARLY = !COSMO || sizeof(R) == 4;
 
     if (active) {
         double nxt[NV];
-        {
-            const long q0 = base + (long)(s0 - 3) * s_ax;
-            nxt[VP] = B.in[0][q0]; nxt[VR] = B.in[1][q0];
-            nxt[VU] = B.in[D::U][q0]; nxt[VV] = B.in[D::V][q0]; nxt[VW] = B.in[D::W][q0];
-            if (GRAV) nxt[NV - 1] = -B.gforce[3 * q0 + (DIR - 1)];
-        }
-        if constexpr (!DEFER) {     // the first cell too, so the loop head holds no wait
+        auto load = [&](long c) {
+            nxt[VP] = at(B.in[0], c); nxt[VR] = at(B.in[1], c);
+            nxt[VU] = at(B.in[D::U], c); nxt[VV] = at(B.in[D::V], c); nxt[VW] = at(B.in[D::W], c);
+            if (GRAV) nxt[NV - 1] = -at(B.gforce, 3 * c + (DIR - 1));
+        };
+        // Take delivery of loads here, not at their first use (the empty asm is
+        // a use): vmcnt counts stores as well, so a wait at the loop's head
+        // would also be for the stores issued just before it.
+        auto deliver = [&]() {
 #pragma unroll
             for (int s = 0; s < NV; ++s) asm volatile("" : "+v"(nxt[s]));
-        }
-        for (int kk = s0 - 3; kk <= s1 + 2; ++kk) {
-            const long q = base + (long)kk * s_ax;
-            double cur[NV];
+        };
+        load(base + (long)(s0 - 3) * s_ax);
+        if constexpr (EARLY) deliver();
+        for (int it = 0; ; ++it) {
+            const int kk = s0 - 3 + it;
+            if (kk > s1 + 2) break;
+            long q = base + (long)kk * s_ax;
+            asm("" : "+v"(q));
+            const long qn = q + (kk < s1 + 2 ? s_ax : 0);   // (the last iteration loads its own cell again)
+            double cur[NV], w3[NV], w2[NV];              // cells k, k-1, k-2
+            {
+                double* const c0 = cell(it);
+                const double* const c1 = cell(it - 1);
+                const double* const c2 = cell(it - 2);
 #pragma unroll
-            for (int s = 0; s < NV; ++s) cur[s] = nxt[s];
-            if (DEFER && kk >= s0 + 4) store_pending(kk - 4);
-            if (kk + 1 <= s1 + 2) {                    // prefetch the next cell of the pencil
-                const long qn = q + s_ax;
-                nxt[VP] = B.in[0][qn]; nxt[VR] = B.in[1][qn];
-                nxt[VU] = B.in[D::U][qn]; nxt[VV] = B.in[D::V][qn]; nxt[VW] = B.in[D::W][qn];
-                if (GRAV) nxt[NV - 1] = -B.gforce[3 * qn + (DIR - 1)];
+                for (int s = 0; s < NV; ++s) {
+                    cur[s] = nxt[s];
+                    w3[s] = c1[s * STREAM_BLOCK];
+                    w2[s] = c2[s * STREAM_BLOCK];
+                    c0[s * STREAM_BLOCK] = cur[s];       // over cell k-4
+                }
             }
+            if constexpr (EARLY) load(qn);
 
             R d3[NV];
             double iv1[NV];
@@ -689,86 +769,98 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
 #pragma unroll
             for (int s = 0; s < NV; ++s) iv1[s] = M::iface(w2[s], w3[s], d2[s], d3[s]);
 
+            const double* const w1 = cell(it - 3);                    // cell k-3
+            const double w1r = w1[VR * STREAM_BLOCK];
             Face<double> fL = fRprev, fR = fRprev;
-            const int ic = kk - 2;                                   // cell k-2, interface at its left
             if (kk >= s0 + 1) {     // parabola and faces of cell k-2
                 int nclL = 0, nclR = 0;
                 const bool flat = flat_always || bits != 0u || bk;
-                M::template cell_faces<R, NV, GRAV, COSMO>(A, w2, iv2, iv1, w0[VR], w1[VR], w3[VR], cur[VR], d1[VR],
-                                                           d3[VR], w1[VP], w3[VP], flat, fL, fR, nclL, nclR);
+                M::template cell_faces<R, NV, GRAV, COSMO>(A, w2, iv2, iv1, w0r, w1r, w3[VR], cur[VR], d1r, d3[VR],
+                                                           w1[VP * STREAM_BLOCK], w3[VP], flat, fL, fR, nclL, nclR);
                 // clamps once per interface of the pencil (0 .. Nax), as the
                 // reference's loop counts them: a segment takes those of its
                 // own cells, the pencil's ends one face beyond
                 if (nclL + nclR) {
-                    if (kk - 2 >= s0 && (kk - 2 < s1 || s1 == Nax)) T.nclamp += nclL;
-                    if ((kk - 2 >= s0 || s0 == 0) && kk - 2 < s1) T.nclamp += nclR;
+                    if (kk - 2 >= s0 && (kk - 2 < s1 || s1 == Nax)) rare[0] += nclL;
+                    if ((kk - 2 >= s0 || s0 == 0) && kk - 2 < s1) rare[0] += nclR;
                 }
             }
-            Flux F = Fprev;
+            Flux F;
+            F.p = F.r = F.u = F.v = F.w = 0.0;
             if (kk >= s0 + 2) {     // Riemann problem at interface k-2
                 int nit;
                 F = M::template riemann<R>(A.Rs, fRprev, fL, nit);
-                peak_floor(A.Rs, F, r5, w0[VR], w1[VR], w2[VR], w0[VU], w1[VU]);
+                // high-density-peak floor (riemannsolver.F90:279-285), the far
+                // cells read again where the near ones ask for them
+                if (w1r > A.Rs.dmax * w2[VR]) {
+                    const long q4 = q - 4 * s_ax;
+                    peak_floor(A.Rs, F, at(B.in[1], q4 - s_ax), at(B.in[1], q4), w1r, w2[VR], at(B.in[D::U], q4),
+                               w1[VU * STREAM_BLOCK]);
+                }
                 // Newton count once per interface of the pencil (0 .. Nax), as
                 // the reference's loop over interfaces: a segment owns
                 // interfaces s0 .. s1-1 and the pencil's last segment also Nax
-                if (kk != s1 + 2 || s1 == Nax) count_newton(nit, T.nitmax, T.nonconv);
+                if (kk != s1 + 2 || s1 == Nax) {
+                    T.nitmax = max(T.nitmax, nit);
+                    if (nit < 0) ++rare[1];
+                }
             }
-            if constexpr (!DEFER) {
-                // take delivery of the prefetch before this cell's stores
-                // (the empty asm is the use; see x_run)
-#pragma unroll
-                for (int s = 0; s < NV; ++s) asm volatile("" : "+v"(nxt[s]));
-            }
+            if constexpr (EARLY) deliver();
+            else load(qn);
             if (kk >= s0 + 3) {     // update cell k-3
-                double pres = w1[VP], rho = w1[VR], u = w1[VU], vv = w1[VV], w = w1[VW];
+                Flux Fprev;
+                Fprev.p = flux[0]; Fprev.r = flux[STREAM_BLOCK]; Fprev.u = flux[2 * STREAM_BLOCK];
+                Fprev.v = flux[3 * STREAM_BLOCK]; Fprev.w = flux[4 * STREAM_BLOCK];
+                double pres = w1[VP * STREAM_BLOCK], rho = w1r, u = w1[VU * STREAM_BLOCK];
+                double vv = w1[VV * STREAM_BLOCK], w = w1[VW * STREAM_BLOCK];
                 const double etot = total_phys<DIR>(A.rgamma1, pres, rho, u, vv, w);
-                M::integrate(A.Is, Fprev, F, pres, rho, u, vv, w, etot, GRAV ? w1[NV - 1] : 0.0, GRAV);
-                pend[0] = pres; pend[1] = rho; pend[D::U] = u; pend[D::V] = vv; pend[D::W] = w;
-                settle_cell<M, EXP>(E, A.gamma, q - 3 * s_ax, pend, T);
-                if (!DEFER) store_pending(kk - 3);
+                M::integrate(A.Is, Fprev, F, pres, rho, u, vv, w, etot, GRAV ? w1[(NV - 1) * STREAM_BLOCK] : 0.0,
+                             GRAV);
+                double val[5];
+                val[0] = pres; val[1] = rho; val[D::U] = u; val[D::V] = vv; val[D::W] = w;
+                const int ic = nb + kk - 3;
+                finish_cell<M, EXP>(B, E, A.gamma, q - 3 * s_ax, val, ixc, DIR == 2 ? ic : ibc, DIR == 2 ? ibc : ic, T);
             }
-            // slide the window
-            r5 = w0[VR];
+            flux[0] = F.p; flux[STREAM_BLOCK] = F.r; flux[2 * STREAM_BLOCK] = F.u;
+            flux[3 * STREAM_BLOCK] = F.v; flux[4 * STREAM_BLOCK] = F.w;
+            // slide the rest of the window
+            w0r = w1r;
+            d1r = d2[VR];
 #pragma unroll
-            for (int s = 0; s < NV; ++s) {
-                w0[s] = w1[s]; w1[s] = w2[s]; w2[s] = w3[s]; w3[s] = cur[s];
-                d1[s] = d2[s]; d2[s] = d3[s]; iv2[s] = iv1[s];
-            }
+            for (int s = 0; s < NV; ++s) { d2[s] = d3[s]; iv2[s] = iv1[s]; }
             bits = (bits >> 1) | ((bk ? 1u : 0u) << 2);
             fRprev = fR;
-            Fprev = F;
         }
-        if (DEFER && s1 + 2 >= s0 + 3) store_pending(s1 - 1);   // the last cell, updated at kk = s1 + 2
     }
 }
 
-// Waves per SIMD a y/z kernel is built for.  Two for gamma = 5/3 and the mixed
-// forms, held there where the allocator would take a register or two over the
-// 256 they allow (gamma = 5/3 FP64 with gravity); the general-gamma FP64
-// forms, and its mixed one with gravity, would spill and keep one.
-template <class M, class R, bool GRAV> constexpr int stream_waves()
+// Waves per SIMD a y/z kernel is built for: what LDS holds of its window
+// (three blocks of 53 KB per CU, two of 61 KB with gravity), and the registers
+// left after it (at most 168 for three waves: the general-gamma and the
+// reference-order forms need 175 to 237).
+template <class M, class R, bool GRAV, bool COSMO> constexpr int stream_waves()
 {
-    return (M::G53 || (sizeof(R) == 4 && !GRAV)) ? 2 : 1;
+    return M::G53 && !GRAV && (COSMO || sizeof(R) == 4) ? 3 : 2;
 }
 
 template <class M, class R, int DIR, bool GRAV, bool COSMO, bool EXP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, GRAV>())))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, GRAV, COSMO>())))
 sweep_stream(BoxView B, Epilogue E, int seglen, int nseg)
 {
+    __shared__ double window[stream_lds<GRAV>() * STREAM_BLOCK];
     if (EXP) load_factors(E);
     int Nax, Nbb;
     long s_ax, s_b;
     stream_geometry<DIR>(B, Nax, Nbb, s_ax, s_b);
-    const long npen = (long)(B.nx - 2 * B.nb) * Nbb;
-    const unsigned tid = blockIdx.x * blockDim.x + threadIdx.x;   // items per sweep < 2^31
-    const bool active = (long)tid < npen * nseg;
-    const unsigned tt = active ? tid : 0u;
-    const int seg = (int)(tt / (unsigned)npen);
-    const long pen = (long)(tt - (unsigned)seg * (unsigned)npen);
-    const AllScalars<R> A = load_scalars<M, R>(B.prm, B.st);
+    const unsigned wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
+    unsigned pen, seg;
+    const bool active = stream_item(wave, (unsigned)((B.nx - 2 * B.nb) * Nbb), pen, seg) && (int)seg < nseg;
+    const AllScalars<R> A = wave_uniform(load_scalars<M, R>(B.prm, B.st));
     Tally T = tally0();
-    stream_run<M, R, DIR, GRAV, COSMO, EXP>(B, A, E, pen, seg, seglen, active, T);
+    double* const column = window + threadIdx.x;
+    reset_rare<GRAV>(column);
+    stream_run<M, R, DIR, GRAV, COSMO, EXP>(B, A, E, pen, seg, seglen, active, T, column);
+    take_rare<GRAV>(column, T);
     flush_counters_block(B.st, T, E.do_speed != 0);
 }
 
@@ -803,12 +895,12 @@ static hipError_t launch_sweep_t(const BoxView& b, const SweepLaunch& L, hipStre
         int seglen = L.seglen;
         if (seglen <= 0) {
             const long npen = (long)Nx * Nbb;
-            const int slots = STREAM_SLOTS * stream_waves<M, R, G>();
-            seglen = stream_seglen(Nax, slots, [&](int nseg) { return (npen * nseg + 63) / 64; });
+            const int slots = STREAM_SLOTS * stream_waves<M, R, G, C>();
+            seglen = stream_seglen(Nax, slots, [&](int nseg) { return stream_items(npen, nseg); });
         }
         if (seglen > Nax) seglen = Nax;
         const int nseg = (Nax + seglen - 1) / seglen;
-        const long threads = (long)Nx * Nbb * nseg;
+        const long threads = stream_items((long)Nx * Nbb, nseg) * 64;
         const long grid = (threads + block - 1) / block;
         if (L.dir == 2)
             hipLaunchKernelGGL((sweep_stream<M, R, 2, G, C, X>), dim3((unsigned)grid), dim3(block), 0, s, b, E,

@@ -178,7 +178,7 @@ int hp_evolve_cosmo(hp_ctx* ctx, int first_step, int nsteps, hp_cosmo* s);
 
 /* Launch shape of this context's sweeps: x_chunks = 58-cell chunks each
  * x-sweep wave walks (0: 16, fewer for small boxes), yz_seglen =
- * y/z pencil segment length (0: at most 64 cells, shorter where the box
+ * y/z pencil segment length (0: at most 24 cells, shorter where the box
  * would not fill the GPU), block = threads per block
  * (0: 256; a multiple of 64, at most 256).  The shape never changes a result.
  * No reference counterpart (the reference's OpenACC gang/vector shapes are
@@ -248,7 +248,7 @@ typedef struct hp_batch_tuning {
     int x_chunks;         /* x sweep: 58-cell chunks per work unit (0: 4) */
     int yz_segments;      /* y/z sweeps: segments each pencil is split into (0: as many as the boxes
                              present need to fill the GPU) */
-    int waves_per_cu;     /* persistent grid: waves per compute unit (0: 8) */
+    int waves_per_cu;     /* persistent grid: waves per compute unit at most (0: as many as fit) */
     int reserved;
 } hp_batch_tuning;
 
