@@ -16,6 +16,7 @@ import numpy as np
 
 from . import _capi
 from ._capi import HpCosmo, check
+from .hydro import field_arrays
 
 _D, _I, _P = ctypes.c_double, ctypes.c_int, ctypes.c_void_p
 _I64, _U64, _SZ = ctypes.c_int64, ctypes.c_uint64, ctypes.c_size_t
@@ -153,7 +154,7 @@ class Batch:
         check("hp_batch_set_newton_limit", self.L.hp_batch_set_newton_limit(self._h, int(i), int(nmax)))
 
     def download(self, i):
-        out = {k: np.zeros(self.shapes[i], dtype=np.float64, order="F") for k in FIELDS}
+        out = field_arrays(self.shapes[i])
         check("hp_batch_download", self.L.hp_batch_download(self._h, int(i),
                                                             *[out[k].ctypes.data_as(_P) for k in FIELDS]))
         return out
@@ -220,7 +221,7 @@ def serve(requests, hbm_budget=64 << 30, max_boxes=64, use_graph=True, keep_fiel
         ptrs = (_P * (5 * nreq))()
         for i in keep_fields:
             n = requests[i]["n"] + 6
-            fields[i] = {k: np.zeros((n, n, n), dtype=np.float64, order="F") for k in FIELDS}
+            fields[i] = field_arrays((n, n, n))
             for j, k in enumerate(FIELDS):
                 ptrs[5 * i + j] = fields[i][k].ctypes.data
     check("hp_serve_run", L.hp_serve_run(arr, nreq, int(hbm_budget), int(max_boxes), 1 if use_graph else 0, ptrs,

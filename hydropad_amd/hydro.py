@@ -29,6 +29,15 @@ def _ptr(a):
     return a.ctypes.data_as(ctypes.c_void_p)
 
 
+def field_arrays(shape):
+    """Five Fortran-ordered (nx, ny, nz) arrays, zero, in one allocation: of a
+    few MB and more it is in huge pages, where first touching the small pages
+    of separate arrays took longer than the copy from the GPU (eight boxes of
+    32^3 to 64^3, 50 MB: 13.0 -> 6.9 ms)."""
+    block = np.zeros((len(FIELDS),) + tuple(shape)[::-1])
+    return {k: block[i].T for i, k in enumerate(FIELDS)}
+
+
 def nrot_of_step(nstep):
     """Sweep-order index of step nstep (hydropad/evolve_sys.F90:30-31)."""
     return 1 if nstep == 1 else nstep % 6 + 1
@@ -118,7 +127,7 @@ class Box:
         check("hp_upload_gforce", self.L.hp_upload_gforce(self._h, _ptr(g) if g is not None else None))
 
     def download(self):
-        out = {k: np.empty(self.shape, dtype=np.float64, order="F") for k in FIELDS}
+        out = field_arrays(self.shape)
         check("hp_download", self.L.hp_download(self._h, *[_ptr(out[k]) for k in FIELDS]))
         return out
 
