@@ -29,17 +29,13 @@ namespace hp {
 namespace fm {
 
 // ---- primitives ------------------------------------------------------------
-// v_rcp_f64 and v_rsq_f64 are accurate to 2^-24 on gfx950 (2^-24.4 and
-// 2^-24.2 measured over 2^-20 .. 2^20), so one third-order step reaches full
-// precision in fewer operations than two Newton steps and rounds no worse:
-// largest error in units of 2^-53, rcp 1.00 (two Newton steps 1.00), rsq 1.25
-// (2.13), x rsq(x) 1.93 (2.81), fsqrt 1.00.  (The Riemann
-// solver's roots stay as they were, see rsq_sqrt_newton.)
 __device__ __forceinline__ double rcp(double b)
 {
-    const double r = __builtin_amdgcn_rcp(b);
-    const double e = fma(-b, r, 1.0);
-    return fma(r, fma(e, e, e), r);
+    double r = __builtin_amdgcn_rcp(b);
+    double e = fma(-b, r, 1.0);
+    r = fma(e, r, r);
+    e = fma(-b, r, 1.0);
+    return fma(e, r, r);
 }
 __device__ __forceinline__ float rcp(float b) { return __builtin_amdgcn_rcpf(b); }
 
@@ -57,8 +53,8 @@ __device__ __forceinline__ double div(double a, double b)
 __device__ __forceinline__ float div(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
 
 // sqrt for x >= 0 without the range scaling of the correctly-rounded
-// expansion: rsq seed, one Goldschmidt step and one correction (within 1 ulp
-// for normal x; 0 for x == 0).
+// expansion: rsq seed and two Goldschmidt corrections (within 1 ulp for
+// normal x; 0 for x == 0).
 __device__ __forceinline__ double fsqrt(double x)
 {
     const double y = __builtin_amdgcn_rsq(x);
@@ -66,29 +62,17 @@ __device__ __forceinline__ double fsqrt(double x)
     const double r = fma(-g, h, 0.5);
     g = fma(g, r, g);
     h = fma(h, r, h);
-    const double d = fma(-g, g, x);
+    double d = fma(-g, g, x);
+    g = fma(d, h, g);
+    d = fma(-g, g, x);
     g = fma(d, h, g);
     return x > 0.0 ? g : 0.0;
 }
 __device__ __forceinline__ float fsqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 
-// 1/sqrt(x) and sqrt(x) for x > 0 together: v_rsq_f64 seed y and one
-// third-order step, y + y e (1/2 + 3/8 e) with e = 1 - x y^2.
+// 1/sqrt(x) and sqrt(x) for x > 0 together: v_rsq_f64 seed and two Newton
+// steps on 1/sqrt, y <- y (1.5 - 0.5 x y^2).
 __device__ __forceinline__ void rsq_sqrt(double x, double& rs, double& sq)
-{
-    const double y = __builtin_amdgcn_rsq(x);
-    const double e = fma(-(x * y), y, 1.0);
-    rs = fma(y * e, fma(0.375, e, 0.5), y);
-    sq = x * rs;
-}
-
-// The same by two Newton steps, y <- y (1.5 - 0.5 x y^2), for the Riemann
-// solver.  The faint leading edge of a wave decides there between patterns on
-// differences of an ulp or so, and a decision the other way shows: of 800 Sod
-// tubes of 32 to 96 cells stepped 40 times, 28 ended further than 1e-11 (none
-// further than 1e-9) from the reference-order form with these, 54 (2) with the
-// third-order step above.
-__device__ __forceinline__ void rsq_sqrt_newton(double x, double& rs, double& sq)
 {
     double y = __builtin_amdgcn_rsq(x);
     y = y * fma(-0.5 * (x * y), y, 1.5);
@@ -492,10 +476,10 @@ __device__ __forceinline__ bool pcheck_guess(const RScal& Rs, double pleft, doub
 
 // One side of the van Leer iteration at pstar (riemann.F90:70-97): the inverse
 // wave impedance 1/a and the left side's form of dv*/dp* (the right side's is
-// its negative).  shock = pstar >= p_side; rc = 1/c for the side's
+// its negative).  shock = pstar >= p_side; cl2 = c^2, rc = 1/c for the side's
 // Lagrangian sound speed c; x = pstar/p_side, xinv = p_side/pstar.
 __device__ __forceinline__ void newton_side(const RScal& Rs, bool shock, double x, double pstar, double pside,
-                                            double rc, double& ra, double& vp)
+                                            double cl2, double rc, double& ra, double& vp)
 {
     const double m = Rs.m, gf = Rs.gf;
     double w = 1.0, wx = 0.0;                        // x^m and x^m / x
@@ -511,9 +495,9 @@ __device__ __forceinline__ void newton_side(const RScal& Rs, bool shock, double 
     if (shock) {                                     // a = c sqrt(gf x + m), v' = -(a^2 + c^2)/(2 a^3)
         const double q = fma(gf, x, m);
         double rs, sq;
-        rsq_sqrt_newton(q, rs, sq);
+        rsq_sqrt(q, rs, sq);
         ra = rc * rs;
-        vp = fma(q, -0.5, -0.5) * (rs * rs) * ra;      // c^2 ra^2 = rs^2
+        vp = -(cl2 * q + cl2) * 0.5 * (ra * ra * ra);
     } else {                                         // a = m c (1 - x)/(1 - x^m), v' = -(1/c) x^m / x
         ra = (1.0 - w) * rcp(m * (1.0 - x)) * rc;
         vp = -rc * wx;
@@ -525,15 +509,17 @@ __device__ __forceinline__ void newton_side(const RScal& Rs, bool shock, double 
 // until the relative change is within terr and returns the iterations done,
 // or -1 past the reference's limit (where riemann.F90:60-65 stops).  vstar
 // is the reference's (pl - pr + a vl + b vr)/(a + b) with the last
-// iteration's impedances, written with 1/a and 1/b.  rcl/rcr are the inverses
-// of the two sides' Lagrangian sound speeds sqrt(gamma p rho)
-// (riemann.F90:68-69).
+// iteration's impedances, written with 1/a and 1/b.  cleft/cright are the
+// Lagrangian sound speeds sqrt(gamma p rho) of the two sides
+// (riemann.F90:68-69), rcl/rcr their inverses.
 // The loop's limit is the reference's constant nnewtmax = 100; a different
 // limit set through the API enters as a head start of the counter
 // (Rs.nskip = 100 - limit), which keeps a runtime bound out of the loop.
 __device__ __forceinline__ int newton(const RScal& Rs, double& pstar, double& vstar, double pleft, double pright,
-                                      double vxleft, double vxright, double rcl, double rcr)
+                                      double vxleft, double vxright, double cleft, double rcl, double cright,
+                                      double rcr)
 {
+    const double cl2 = cleft * cleft, cr2 = cright * cright;
     const double rpl = rcp(pleft), rpr = rcp(pright);
     double ra = 0.0, rb = 0.0;
     int k = Rs.nskip;
@@ -544,8 +530,8 @@ __device__ __forceinline__ int newton(const RScal& Rs, double& pstar, double& vs
         }
         const double pstarold = pstar;
         double vpl, vpr;
-        newton_side(Rs, pstar >= pleft, pstar * rpl, pstar, pleft, rcl, ra, vpl);
-        newton_side(Rs, pstar >= pright, pstar * rpr, pstar, pright, rcr, rb, vpr);
+        newton_side(Rs, pstar >= pleft, pstar * rpl, pstar, pleft, cl2, rcl, ra, vpl);
+        newton_side(Rs, pstar >= pright, pstar * rpr, pstar, pright, cr2, rcr, rb, vpr);
         const double vstarl = vxleft - (pstar - pleft) * ra;
         const double vstarr = vxright + (pstar - pright) * rb;
         // the step (vprimel - vprimer = vpl + vpr) with one Newton step on the
@@ -604,15 +590,15 @@ __device__ __forceinline__ void riemann_setup(const RScal& Rs, const Face<double
     // Newton iteration's Lagrangian C = rho c and 1/C = (1/c)(1/rho) follow
     S.rrl = rcp(rholeft);
     S.rrr = rcp(rhoright);
-    rsq_sqrt_newton(gamma * pleft * S.rrl, S.rcle, S.cleft);
-    rsq_sqrt_newton(gamma * pright * S.rrr, S.rcre, S.cright);
+    rsq_sqrt(gamma * pleft * S.rrl, S.rcle, S.cleft);
+    rsq_sqrt(gamma * pright * S.rrr, S.rcre, S.cright);
     const double cleft = S.cleft, cright = S.cright;
     R p1, p2, rho1, c1, c2;
     if (pleft <= pright) { p1 = pleft; p2 = pright; rho1 = rholeft; c1 = cleft; c2 = cright; }
     else { p1 = pright; p2 = pleft; rho1 = rhoright; c1 = cright; c2 = cleft; }
     const R dvv = vxleft - vxright;
     double rs2, sq2;
-    rsq_sqrt_newton(R(0.5) * rho1 * ((gamma - R(1)) * p1 + (gamma + R(1)) * p2), rs2, sq2);
+    rsq_sqrt(R(0.5) * rho1 * ((gamma - R(1)) * p1 + (gamma + R(1)) * p2), rs2, sq2);
     const R dv2s = (p2 - p1) * rs2;
     const R dv2r = -R(2) * (c1 + c2) * rgamma1;
     int kase;
@@ -642,7 +628,8 @@ __device__ __forceinline__ void riemann_setup(const RScal& Rs, const Face<double
 __device__ __forceinline__ void riemann_newton(const RScal& Rs, const Face<double>& L, const Face<double>& Rt,
                                                RSolve& S)
 {
-    S.nit = fm::newton(Rs, S.pm, S.vxm, L.p, Rt.p, L.u, Rt.u, S.rcle * S.rrl, S.rcre * S.rrr);
+    S.nit = newton(Rs, S.pm, S.vxm, L.p, Rt.p, L.u, Rt.u, L.r * S.cleft, S.rcle * S.rrl, Rt.r * S.cright,
+                   S.rcre * S.rrr);
 }
 
 // The costly sampling operations in precision Q.  Q = double: the FP64
