@@ -320,6 +320,31 @@ __device__ __forceinline__ R beta_source_d(const SweepScalars<R>& S, R rct, R pc
     return beta_sum_d<R, GRAV, COSMO>(S, R(0), rct, pc_abs, uc_abs, gc_abs, sign);
 }
 
+// Average of a parabola's offset over a distance x dx from its right or left
+// edge (ppm_functs.F90:91-124), with each operation's fusing written out: the
+// tracing forms the averages on either side of branches, where the compiler's
+// own choice of what to fuse changes with the code around them, and with it
+// the FP32 form's result by 1e-10 to 1e-9.  The transverse velocities take one of two
+// averages by a sign, so their last operation stands after the choice and is
+// not fused: trace_step is their average's distance from the edge.
+__device__ __forceinline__ float fma_r(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double fma_r(double a, double b, double c) { return __builtin_fma(a, b, c); }
+template <class R, bool RIGHT> __device__ __forceinline__ R trace_slope(const Parab<R>& q, R x)
+{
+    const R w = fma_r(-(R(2) * x), R(K_THIRD), R(1));
+    return RIGHT ? fma_r(-w, q.a6, q.d) : fma_r(w, q.a6, q.d);
+}
+template <class R, bool RIGHT> __device__ __forceinline__ R trace_d(const Parab<R>& q, R x)
+{
+    return fma_r((RIGHT ? R(-0.5) : R(0.5)) * x, trace_slope<R, RIGHT>(q, x), RIGHT ? q.r : q.l);
+}
+template <class R, bool RIGHT> __device__ __forceinline__ R trace_step(const Parab<R>& q, R x)
+{
+    R s = (RIGHT ? R(-0.5) : R(0.5)) * x * trace_slope<R, RIGHT>(q, x);
+    asm("" : "+v"(s));                                   // rounded here, not fused into the sum
+    return s;
+}
+
 // Traced face state of a cell.  RIGHT = true: its right face (the
 // reference's left state of interface c+1/2, fl of the parabola at the
 // characteristics u+c, u, u-c, ppm_functs.F90:59-75, order2interp.F90:192-219);
@@ -343,10 +368,10 @@ __device__ __forceinline__ Face<double> trace_face_d(const SweepScalars<R>& S, c
         x2 = -(R)u0 * k;
         x3 = -(R)up * k;
     }
-    auto tr = [&](const Parab<R>& p, R x) { return RIGHT ? pfl(p, x) : pfr(p, x); };
+    auto tr = [&](const Parab<R>& p, R x) { return trace_d<R, RIGHT>(p, x); };
     auto gravity = [&](R x) { return GRAV ? (R)a[VG] + tr(q[VG], x) : R(0); };
     R pt = tr(q[VP], xt), rt = tr(q[VR], xt);
-    const R ut = tr(q[VU], xt), vt = tr(q[VV], xt), wt = tr(q[VW], xt);
+    const R ut = tr(q[VU], xt);
     double ptl = a[VP] + (double)pt, rtl = a[VR] + (double)rt;
     const bool pneg = ptl < 0.0;
     if (pneg) { ptl = K_1EM15; pt = (R)(K_1EM15 - a[VP]); ++nclamp; }
@@ -365,7 +390,7 @@ __device__ __forceinline__ Face<double> trace_face_d(const SweepScalars<R>& S, c
     Face<double> f;
     f.p = ptl;
     f.r = rtl;
-    R vf = vt, wf = wt, du = ut;
+    R du = ut;
     if (GRAV || COSMO || away || pneg) {
         // the Lagrangian sound speed and its inverse (order2interp.F90:192-193):
         // in FP64 both from one rsq; in FP32 the hardware root and reciprocal
@@ -400,8 +425,6 @@ __device__ __forceinline__ Face<double> trace_face_d(const SweepScalars<R>& S, c
             const R rtr = (R)rtl, rcr = (R)a[VR] + rc2;
             b0 = (pt - pc2) * rct2 + div(rc2 - rt, rtr * rcr);
             if (COSMO) b0 = b0 + S.cdat2 * (ap + pc2) * rct2;                 // 2 adot pc dt/(a C^2)
-            vf = tr(q[VV], x2);
-            wf = tr(q[VW], x2);
         }
         const R bp = RIGHT ? bo : bi, bm = RIGHT ? bi : bo;
         f.p = ptl + (double)(ct * ct * (bp + bm));
@@ -417,9 +440,90 @@ __device__ __forceinline__ Face<double> trace_face_d(const SweepScalars<R>& S, c
         if (f.r <= 0.0) f.r = rtl;
     }
     f.u = a[VU] + (double)du;
+    const R xv = away ? x2 : xt;
+    f.v = a[VV] + (double)((RIGHT ? q[VV].r : q[VV].l) + trace_step<R, RIGHT>(q[VV], xv));
+    f.w = a[VW] + (double)((RIGHT ? q[VW].r : q[VW].l) + trace_step<R, RIGHT>(q[VW], xv));
+    return f;
+}
+
+// The FP32 form without gravity or expansion keeps every average formed and
+// its fusing the compiler's: the rounding of the outermost wave's vanishing
+// differences is part of its result (6e-10 to 9e-9 of a y/z sweep), and the
+// branches of trace_face_d gained it nothing (512x512x64, 4 steps: 17.8 ms
+// with either).
+template <class R, bool RIGHT>
+__device__ __forceinline__ Face<double> trace_face_plain(const SweepScalars<R>& S, const Parab<R>* q, const double* a,
+                                                     double cs, double gamma, int& nclamp)
+{
+    const double um = a[VU] - cs, u0 = a[VU], up = a[VU] + cs;     // characteristic speeds (FP64 signs)
+    const R k = S.ktrace;
+    R xt, x1, x2, x3;
+    if (RIGHT) {
+        x3 = (R)up * k;
+        xt = tmax(x3, R(0));
+        x1 = (R)um * k;
+        x2 = (R)u0 * k;
+    } else {
+        x1 = -(R)um * k;
+        xt = tmax(x1, R(0));
+        x2 = -(R)u0 * k;
+        x3 = -(R)up * k;
+    }
+    auto tr = [&](const Parab<R>& p, R x) { return RIGHT ? pfl(p, x) : pfr(p, x); };
+    R pt = tr(q[VP], xt), rt = tr(q[VR], xt), ut = tr(q[VU], xt), vt = tr(q[VV], xt), wt = tr(q[VW], xt);
+    const R pc1 = tr(q[VP], x1), pc2 = tr(q[VP], x2), pc3 = tr(q[VP], x3);
+    const R rc2 = tr(q[VR], x2), uc1 = tr(q[VU], x1), uc3 = tr(q[VU], x3);
+    const R vc2 = tr(q[VV], x2), wc2 = tr(q[VW], x2);
+    double ptl = a[VP] + (double)pt, rtl = a[VR] + (double)rt;
+    if (ptl < 0.0) { ptl = K_1EM15; pt = (R)(K_1EM15 - a[VP]); ++nclamp; }
+    if (rtl < 0.0) { rtl = K_1EM15; rt = (R)(K_1EM15 - a[VR]); ++nclamp; }
+    const R ct = fsqrt((R)(gamma * ptl * rtl)), rct = rcp(ct);
+    const R ap = (R)a[VP], au = (R)a[VU];
+    R bm = R(0), bp = R(0), b0 = R(0);
+    R vf = vt, wf = wt;
+    if (RIGHT) {
+        if (um > 0.0) bm = beta_d<R, false, false>(S, rct, ut, uc1, pt, pc1, ap + pc1, au + uc1, R(0), R(-1));
+        if (up > 0.0) bp = beta_d<R, false, false>(S, rct, ut, uc3, pt, pc3, ap + pc3, au + uc3, R(0), R(1));
+        if (u0 > 0.0) {
+            vf = vc2;
+            wf = wc2;
+        }
+    } else {
+        if (up < 0.0) bp = beta_d<R, false, false>(S, rct, ut, uc3, pt, pc3, ap + pc3, au + uc3, R(0), R(1));
+        if (um < 0.0) bm = beta_d<R, false, false>(S, rct, ut, uc1, pt, pc1, ap + pc1, au + uc1, R(0), R(-1));
+        if (u0 < 0.0) {
+            vf = vc2;
+            wf = wc2;
+        }
+    }
+    if (RIGHT ? (u0 > 0.0) : (u0 < 0.0)) {
+        // beta0 (ppm_functs.F90:149-162) with 1/rho_t - 1/rho_c = (rho_c - rho_t)/(rho_t rho_c)
+        const R rct2 = rct * rct;
+        const R rtr = (R)rtl, rcr = (R)a[VR] + rc2;
+        b0 = (pt - pc2) * rct2 + div(rc2 - rt, rtr * rcr);
+    }
+    Face<double> f;
+    f.p = ptl + (double)(ct * ct * (bp + bm));
+    if (f.p <= 0.0) f.p = ptl;
+    f.u = a[VU] + (double)(ut + ct * (bp - bm));
+    // 1/(1/rho_t - bm - b0 - bp) = rho_t / (1 - rho_t (bm + b0 + bp))
+    // in delta form: rtl + rtl s/(1 - s)
+    const R sb = (R)rtl * (bm + b0 + bp);
+    f.r = rtl + rtl * (double)(sb * rcp(R(1) - sb));
+    if (f.r <= 0.0) f.r = rtl;
     f.v = a[VV] + (double)vf;
     f.w = a[VW] + (double)wf;
     return f;
+}
+
+template <class R, bool GRAV, bool COSMO, bool RIGHT>
+__device__ __forceinline__ Face<double> trace_face(const SweepScalars<R>& S, const Parab<R>* q, const double* a,
+                                                   double cs, double gamma, int& nclamp)
+{
+    if constexpr (sizeof(R) == 4 && !GRAV && !COSMO)
+        return trace_face_plain<R, RIGHT>(S, q, a, cs, gamma, nclamp);
+    else
+        return trace_face_d<R, GRAV, COSMO, RIGHT>(S, q, a, cs, gamma, nclamp);
 }
 
 // Parabolas of one cell and its two traced faces (delta form).
@@ -454,8 +558,8 @@ __device__ __forceinline__ void cell_faces_d(const SweepScalars<R>& S, double ga
         const double c2 = gamma * a[VP] * __builtin_amdgcn_rcp(a[VR]);
         cs = c2 > 0.0 ? c2 * __builtin_amdgcn_rsq(c2) : 0.0;
     }
-    fR = trace_face_d<R, GRAV, COSMO, true>(S, q, a, cs, gamma, nclR);
-    fL = trace_face_d<R, GRAV, COSMO, false>(S, q, a, cs, gamma, nclL);
+    fR = trace_face<R, GRAV, COSMO, true>(S, q, a, cs, gamma, nclR);
+    fL = trace_face<R, GRAV, COSMO, false>(S, q, a, cs, gamma, nclL);
 }
 
 // ---- Riemann solver ------------------------------------------------------------------
@@ -878,8 +982,11 @@ __device__ __forceinline__ void integrate_cell(const IScal& S, const Flux& F1, c
     double px = vx * rho + lam * ((m1 * F1.u + F1.p) - (m2 * F2.u + F2.p));
     if (grav) px += S.rdtath * ((rho + rhonew) * ghalf * 0.5);
     const double vxnew = px * rrn;
-    const double vynew = (rho * vy + lam * (F1.v * m1 - F2.v * m2)) * rrn;
-    const double vznew = (rho * vz + lam * (F1.w * m1 - F2.w * m2)) * rrn;
+    // which product is rounded is written out: left to the compiler, the x and
+    // the y/z sweeps round the transverse momenta differently
+    auto momentum = [&](double r, double v, double d) { return fma(r, v, lam * d); };
+    const double vynew = momentum(rho, vy, F1.v * m1 - F2.v * m2) * rrn;
+    const double vznew = momentum(rho, vz, F1.w * m1 - F2.w * m2) * rrn;
     const double e1 = (gamma * F1.p * rgamma1 + 0.5 * F1.r * (F1.u * F1.u + F1.v * F1.v + F1.w * F1.w)) * F1.u;
     const double e2 = (gamma * F2.p * rgamma1 + 0.5 * F2.r * (F2.u * F2.u + F2.v * F2.v + F2.w * F2.w)) * F2.u;
     double etotnew = etot + lam * (e1 - e2);
