@@ -183,14 +183,14 @@ int persistent_grid(const hp_batch* b)
     return std::max(1, b->ncu * wpc / 4);
 }
 
-// Work units of a box: x chunks per unit from the tuning, y/z segments from
-// it too or, where it leaves them open, of at most `len` cells.
-void set_units(hp::BatchBox& X, const hp_batch_tuning& t, int len)
+// Work units of a box: x chunks per unit and y/z segments from the tuning or,
+// where it leaves them open, `chunks` and segments of at most `len` cells.
+void set_units(hp::BatchBox& X, const hp_batch_tuning& t, int chunks, int len)
 {
     const int Nx = X.nx - 2 * X.nb, Ny = X.ny - 2 * X.nb, Nz = X.nz - 2 * X.nb;
     const long total = (long)Ny * Nz * X.nx;
     const long nchunks = (total + 57) / 58;
-    X.xcpu = t.x_chunks > 0 ? t.x_chunks : 4;
+    X.xcpu = t.x_chunks > 0 ? t.x_chunks : chunks;
     X.units[0] = (int)((nchunks + X.xcpu - 1) / X.xcpu);
     for (int d = 0; d < 2; ++d) {
         const int Nax = d == 0 ? Ny : Nz;
@@ -223,16 +223,22 @@ int push_box(hp_batch* b, int id)
 }
 
 // Work units of every active box, before a step that follows a change of the
-// boxes or of the tuning.  The segment length a tuning leaves open is one for
-// the whole batch, by the rule of the single-box sweeps (stream_seglen) on
-// the waves of all boxes against those of the persistent grid.  Eight
-// comoving boxes of 32^3 to 64^3, 40 steps with their uploads and downloads:
-// 57.5 ms with whole pencils, 30.1 ms with this rule.
+// boxes or of the tuning.  What a tuning leaves open is one for the whole
+// batch, by the rules of the single-box sweeps (x_chunks_per_wave,
+// stream_seglen) on all boxes' chunks and waves, these against the waves of
+// the persistent grid.  Eight comoving boxes of 32^3 to 64^3, 40 steps with
+// their uploads and downloads: 57.5 ms with whole pencils, 30.1 ms with this
+// rule, 25 ms with the window in LDS.
 int tile_boxes(hp_batch* b)
 {
     int nax = 1;
+    long nchunks = 0;
     for (const hp::BatchBox& X : b->h_boxes)
-        if (X.active) nax = std::max(nax, std::max(X.ny, X.nz) - 2 * X.nb);
+        if (X.active) {
+            nax = std::max(nax, std::max(X.ny, X.nz) - 2 * X.nb);
+            nchunks += ((long)(X.ny - 2 * X.nb) * (X.nz - 2 * X.nb) * X.nx + 57) / 58;
+        }
+    const int chunks = hp::x_chunks_per_wave(nchunks);
     const int slots = 4 * std::min(persistent_grid(b), 3 * b->ncu);   // waves of a y/z sweep's grid
     const int len = hp::stream_seglen(nax, slots, [&](int nseg) {
         const int l = (nax + nseg - 1) / nseg;
@@ -245,7 +251,7 @@ int tile_boxes(hp_batch* b)
         return waves;
     });
     for (hp::BatchBox& X : b->h_boxes)
-        if (X.active) set_units(X, b->tune, len);
+        if (X.active) set_units(X, b->tune, chunks, len);
     if (b->nbox > 0)
         HPCHK(hipMemcpyAsync(b->d_boxes, b->h_boxes.data(), sizeof(hp::BatchBox) * b->nbox, hipMemcpyHostToDevice,
                              b->stream));

@@ -88,12 +88,9 @@ __global__ void __launch_bounds__(256) batch_x(const BatchBox* __restrict__ boxe
     if (cur >= 0) flush_counters(boxes[cur].st, t, slot == 2);
 }
 
-// At least two waves per SIMD for the gamma = 5/3 forms and the mixed forms:
-// left to itself the allocator gives the 5/3 FP64 z-sweep body 257 registers
-// and the general-gamma mixed bodies 259, just above the 256 that two waves
-// allow, and those kernels run at one wave per SIMD; held at two they fit
-// with no spill.  (The general-gamma FP64 bodies need ~290; forced to two
-// waves they spill about 1 KB per lane, so they are left to the allocator.)
+// Waves per SIMD as the single-box comoving sweeps (stream_waves): three for
+// gamma = 5/3, two else; held there the bodies fit without a spill, left to
+// itself the allocator takes a few registers more and a wave is lost.
 template <class M, class R, int DIR, bool EXP>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, false, true>())))
 batch_stream(const BatchBox* __restrict__ boxes, const BatchPlan* __restrict__ plan, int key, int slot)

@@ -60,7 +60,7 @@ struct SweepLaunch {
     int ghost_mask;   // bit d-1: also write the periodic face-ghost images along axis d
     int do_speed;     // fuse the CFL maximum into this sweep
     int seglen;       // streaming segment length for y/z sweeps (<= 0: stream_seglen)
-    int xcpw;         // x sweep: chunks per wave (<= 0: 16, fewer for small boxes)
+    int xcpw;         // x sweep: chunks per wave (<= 0: x_chunks_per_wave)
     int block;        // threads per block
     int precision;    // Precision
     bool grav, cosmo;
@@ -71,6 +71,21 @@ struct SweepLaunch {
     const double* old[4];
     const double* fac;
 };
+
+// Chunks of 58 cells each wave of an x sweep (or unit of a batch's) walks: one
+// where the box has few, more as it grows, since a wave's first chunk waits for
+// its loads and for the box's scalars; 16 only where even those make 48
+// thousand waves, as short runs balance the Riemann work.  Measured, us at 1,
+// 2, 4, 8, 16: 64^3 comoving [33] 36 47 64 117; 96^3 80 [76] 80 88 121; 128^3
+// 165 [163] 169 177 220; 192^3 516 488 [480] 494 512; 256^3 1190 1119 1088
+// [1094] 1120; 512x512x64 mixed tube 789 714 637 [627] 638; 512x512x256 tube
+// 3978 3494 3004 2938 [2890].
+inline int x_chunks_per_wave(long nchunks)
+{
+    int n = 1;
+    for (long most = 12000; nchunks >= most && n < 16; most *= 4) n *= 2;
+    return n;
+}
 
 // Waves of a y/z sweep the chip holds at once, for each wave its SIMD holds:
 // 256 CUs x 4 SIMDs.

@@ -880,11 +880,7 @@ static hipError_t launch_sweep_t(const BoxView& b, const SweepLaunch& L, hipStre
     if (L.dir == 1) {
         const long total = (long)Ny * Nz * b.nx;
         const long nchunks = (total + 57) / 58;
-        // waves of 16 chunks (fewer for small boxes, to keep ~16K waves):
-        // short runs balance the divergent Riemann work across the chip
-        long cpw = std::min<long>(16, nchunks / 16384);
-        if (L.xcpw > 0) cpw = L.xcpw;
-        if (cpw < 1) cpw = 1;
+        const long cpw = L.xcpw > 0 ? L.xcpw : x_chunks_per_wave(nchunks);
         const long waves = (nchunks + cpw - 1) / cpw;
         const long threads = waves * 64;
         const long grid = (threads + block - 1) / block;

@@ -177,7 +177,7 @@ int hp_expand(hp_ctx* ctx, double afact);
 int hp_evolve_cosmo(hp_ctx* ctx, int first_step, int nsteps, hp_cosmo* s);
 
 /* Launch shape of this context's sweeps: x_chunks = 58-cell chunks each
- * x-sweep wave walks (0: 16, fewer for small boxes), yz_seglen =
+ * x-sweep wave walks (0: 1 to 16, by the box's size), yz_seglen =
  * y/z pencil segment length (0: at most 24 cells, shorter where the box
  * would not fill the GPU), block = threads per block
  * (0: 256; a multiple of 64, at most 256).  The shape never changes a result.
@@ -245,7 +245,7 @@ int hp_sync(hp_ctx* ctx);
 typedef struct hp_batch hp_batch;
 
 typedef struct hp_batch_tuning {
-    int x_chunks;         /* x sweep: 58-cell chunks per work unit (0: 4) */
+    int x_chunks;         /* x sweep: 58-cell chunks per work unit (0: 1 to 16, by the boxes present) */
     int yz_segments;      /* y/z sweeps: segments each pencil is split into (0: as many as the boxes
                              present need to fill the GPU) */
     int waves_per_cu;     /* persistent grid: waves per compute unit at most (0: as many as fit) */
