@@ -124,10 +124,10 @@ batch_stream(const BatchBox* __restrict__ boxes, const BatchPlan* __restrict__ p
         Epilogue E;
         batch_view(X, slot, V, E);
         const int Nbb = (DIR == 2) ? X.nz - 2 * X.nb : X.ny - 2 * X.nb;
-        unsigned pen, seg;
-        const bool active = stream_item((unsigned)local, (unsigned)((X.nx - 2 * X.nb) * Nbb), pen, seg);
+        const StreamItem I = stream_item((unsigned)local, threadIdx.x & 63u, (unsigned)((X.nx - 2 * X.nb) * Nbb),
+                                         (unsigned)X.nseg[DIR - 2]);
         const AllScalars<R> A = wave_uniform(load_scalars<M, R>(X.prm, X.st));
-        stream_run<M, R, DIR, false, true, EXP>(V, A, E, pen, (int)seg, X.seglen[DIR - 2], active, t, column);
+        stream_run<M, R, DIR, false, true, EXP>(V, A, E, I.pen, (int)I.seg, X.seglen[DIR - 2], I.active, t, column);
     }
     if (cur >= 0) {
         take_rare<false>(column, t);

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "hp_tiling.h"
+
 namespace hp {
 
 struct Params;
@@ -71,57 +73,6 @@ struct SweepLaunch {
     const double* old[4];
     const double* fac;
 };
-
-// Chunks of 58 cells each wave of an x sweep (or unit of a batch's) walks: one
-// where the box has few, more as it grows, since a wave's first chunk waits for
-// its loads and for the box's scalars; 16 only where even those make 48
-// thousand waves, as short runs balance the Riemann work.  Measured, us at 1,
-// 2, 4, 8, 16: 64^3 comoving [33] 36 47 64 117; 96^3 80 [76] 80 88 121; 128^3
-// 165 [163] 169 177 220; 192^3 516 488 [480] 494 512; 256^3 1190 1119 1088
-// [1094] 1120; 512x512x64 mixed tube 789 714 637 [627] 638; 512x512x256 tube
-// 3978 3494 3004 2938 [2890].
-inline int x_chunks_per_wave(long nchunks)
-{
-    int n = 1;
-    for (long most = 12000; nchunks >= most && n < 16; most *= 4) n *= 2;
-    return n;
-}
-
-// Waves of a y/z sweep the chip holds at once, for each wave its SIMD holds:
-// 256 CUs x 4 SIMDs.
-constexpr int STREAM_SLOTS = 1024;
-
-// Segment length of a y/z sweep whose pencils are `nax` cells long and take
-// `waves(nseg)` waves when each is split into nseg segments.  A wave walks a
-// segment of len cells in len + 6 iterations, the first four of them cheap:
-// about len + 4 cells' time, and the waves run in rounds of `slots`.  The
-// split with the smallest rounds x (len + 4) is taken, at most 24 cells long:
-// short enough that the waves that got the most Newton iterations do not run
-// on alone, and that the rows two segments share are still in cache.  Measured, y sweep in us, by length (taken one in brackets):
-//   64^3 tube                 64: 155   16: 49   8: 33   [2]: 24
-//   96^3 comoving             48: 353   16: 133  7: 94   [5]: 96   4: 107
-//   128^3 comoving            64: 448   32: 245  16: 174 [11]: 167  10: 181
-//   192^3 comoving            64: 640   28: 503  24: 520 [20]: 475  18: 491
-//   256^3 comoving            64: 1053  32: 1010 24: 984 [22]: 1042 16: 1023
-//   512^3 tube                128: 3270 64: 3132 32: 2995 [20]: 2854 16: 2811
-// A length just past a full round (10 at 128^3, 24 at 192^3) is slower than
-// its neighbours.
-template <class Waves> inline int stream_seglen(int nax, int slots, Waves waves)
-{
-    int best = nax < 24 ? nax : 24;
-    long cost = -1;
-    for (int nseg = (nax + best - 1) / best; nseg <= nax; ++nseg) {
-        const int len = (nax + nseg - 1) / nseg;
-        const long rounds = (waves((nax + len - 1) / len) + slots - 1) / slots;
-        const long c = rounds * (len + 4);
-        if (cost < 0 || c < cost) { cost = c; best = len; }
-        if (rounds * 5 > cost) break;                  // shorter segments only cost more from here
-    }
-    return best;
-}
-
-// Waves of a y/z sweep of npen pencils in nseg segments each (hp_sweep.h).
-inline long stream_items(long npen, int nseg) { return (npen + 255) / 256 * 4 * nseg; }
 
 hipError_t launch_sweep(const BoxView& b, const SweepLaunch& L, hipStream_t s);
 // Periodic ghost fill of the 5 fields of `f` (in place); dir 1..3 or 0 = all (z, x, y).

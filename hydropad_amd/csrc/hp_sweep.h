@@ -8,8 +8,9 @@
 //                  neighbours come from DPP wave shifts.  Lanes 3..60 own
 //                  their output, so a wave advances 58 cells.
 //   sweep_stream   y and z sweeps.  One thread walks a pencil segment along
-//                  the strided axis with a register sliding window; lanes of
-//                  a wave are consecutive x, so every load/store coalesces.
+//                  the strided axis; the window it slides along stands in LDS.
+//                  Lanes of a wave are consecutive x, so every load/store
+//                  coalesces.
 // Both read the source buffer and write the other one (ping-pong), so pencils
 // can be split into segments without a read/write race, and they write the
 // periodic face-ghost images of what they store (the one-rank exchange_mesh,
@@ -628,22 +629,6 @@ template <int DIR> __device__ __forceinline__ void stream_geometry(const BoxView
     else { Nax = B.nz - 2 * nb; Nbb = B.ny - 2 * nb; s_ax = (long)B.nx * B.ny; s_b = B.nx; }
 }
 
-// The work of one of stream_items' waves: a lane per pencil, one segment for
-// all, so that the loop over the segment and its guards are scalar.  Four
-// consecutive waves take 256 consecutive pencils, whose rows are 2 KB of
-// memory, and a segment of all pencils comes before the next (one wave's 512
-// bytes at a time with the segments side by side: 512x512x256 tube 1405 ->
-// 1704 us, 256^3 comoving 1065 -> 1110).
-__device__ __forceinline__ bool stream_item(unsigned wave, unsigned npen, unsigned& pen, unsigned& seg)
-{
-    const unsigned groups = (npen + 255u) >> 8, four = wave >> 2;
-    seg = four / groups;
-    pen = ((four - seg * groups) * 4u + (wave & 3u)) * 64u + (threadIdx.x & 63u);
-    const bool active = pen < npen;
-    if (!active) pen = 0u;
-    return active;
-}
-
 // The window a thread slides along its segment lives in LDS, one column of
 // doubles per thread: a ring of the last four cells and the flux at the
 // interface behind.  Only the thread itself reads its column, so nothing
@@ -690,8 +675,15 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
     long s_ax, s_b;
     stream_geometry<DIR>(B, Nax, Nbb, s_ax, s_b);
     const int ib = (int)(pen / (unsigned)Nx), ia = (int)(pen - (unsigned)ib * (unsigned)Nx);
-    const int s0 = seg * seglen;
-    const int s1 = min(s0 + seglen, Nax);
+    // Every lane runs the iterations of its wave's first segment, the longest,
+    // so that the loop and its guards are scalar also where a wave holds
+    // several: a segment that the pencil's end would cut short starts earlier,
+    // and its first `skip` cells, the segment's before it, are not stored.
+    const int len = min(seglen, Nax - __builtin_amdgcn_readfirstlane(seg) * seglen);
+    const int s0 = min(seg * seglen, Nax - len);   // first cell walked
+    const int skip = seg * seglen - s0;
+    const int s0_wave = __builtin_amdgcn_readfirstlane(s0);
+    const bool alone = stream_pack((unsigned)(Nx * Nbb)) == 1u;   // s0 is s0_wave
     const long base = (nb + ia) + (long)(nb + ib) * s_b + (long)nb * s_ax;   // interior cell 0 of the pencil
     const bool flat_always = A.mingradflat <= 0.0;
 
@@ -729,14 +721,12 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
 #pragma unroll
             for (int s = 0; s < NV; ++s) asm volatile("" : "+v"(nxt[s]));
         };
-        load(base + (long)(s0 - 3) * s_ax);
+        long q = base + (long)(s0 - 3) * s_ax;
+        load(q);
         if constexpr (EARLY) deliver();
-        for (int it = 0; ; ++it) {
-            const int kk = s0 - 3 + it;
-            if (kk > s1 + 2) break;
-            long q = base + (long)kk * s_ax;
-            asm("" : "+v"(q));
-            const long qn = q + (kk < s1 + 2 ? s_ax : 0);   // (the last iteration loads its own cell again)
+        const int last = len + 5;
+        for (int it = 0; it <= last; ++it) {             // k = s0 - 3 + it
+            const long qn = q + (it < last ? s_ax : 0);  // (the last iteration loads its own cell again)
             double cur[NV], w3[NV], w2[NV];              // cells k, k-1, k-2
             {
                 double* const c0 = cell(it);
@@ -755,14 +745,14 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
             R d3[NV];
             double iv1[NV];
             bool bk = false;
-            if (kk >= s0 - 1) {
+            if (it >= 2) {
 #pragma unroll
                 for (int s = 0; s < NV; ++s) d3[s] = M::template slope<R>(w2[s], w3[s], cur[s]);
             } else {
 #pragma unroll
                 for (int s = 0; s < NV; ++s) d3[s] = R(0);
             }
-            if (kk >= s0 - 2) {
+            if (it >= 1) {
 #pragma unroll
                 for (int s = 0; s < 5; ++s) bk |= M::steep(w3[s], cur[s], A.mingradflat);
             }
@@ -772,7 +762,7 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
             const double* const w1 = cell(it - 3);                    // cell k-3
             const double w1r = w1[VR * STREAM_BLOCK];
             Face<double> fL = fRprev, fR = fRprev;
-            if (kk >= s0 + 1) {     // parabola and faces of cell k-2
+            if (it >= 4) {     // parabola and faces of cell k-2
                 int nclL = 0, nclR = 0;
                 const bool flat = flat_always || bits != 0u || bk;
                 M::template cell_faces<R, NV, GRAV, COSMO>(A, w2, iv2, iv1, w0r, w1r, w3[VR], cur[VR], d1r, d3[VR],
@@ -781,13 +771,14 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
                 // reference's loop counts them: a segment takes those of its
                 // own cells, the pencil's ends one face beyond
                 if (nclL + nclR) {
-                    if (kk - 2 >= s0 && (kk - 2 < s1 || s1 == Nax)) rare[0] += nclL;
-                    if ((kk - 2 >= s0 || s0 == 0) && kk - 2 < s1) rare[0] += nclR;
+                    const bool own = it - 5 >= skip;
+                    if (own && (it < last || s0 + len == Nax)) rare[0] += nclL;
+                    if ((own || s0 == 0) && it < last) rare[0] += nclR;
                 }
             }
             Flux F;
             F.p = F.r = F.u = F.v = F.w = 0.0;
-            if (kk >= s0 + 2) {     // Riemann problem at interface k-2
+            if (it >= 5) {     // Riemann problem at interface k-2
                 int nit;
                 F = M::template riemann<R>(A.Rs, fRprev, fL, nit);
                 // high-density-peak floor (riemannsolver.F90:279-285), the far
@@ -797,17 +788,15 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
                     peak_floor(A.Rs, F, at(B.in[1], q4 - s_ax), at(B.in[1], q4), w1r, w2[VR], at(B.in[D::U], q4),
                                w1[VU * STREAM_BLOCK]);
                 }
-                // Newton count once per interface of the pencil (0 .. Nax), as
-                // the reference's loop over interfaces: a segment owns
-                // interfaces s0 .. s1-1 and the pencil's last segment also Nax
-                if (kk != s1 + 2 || s1 == Nax) {
-                    T.nitmax = max(T.nitmax, nit);
-                    if (nit < 0) ++rare[1];
-                }
+                // iterations that did not converge once per interface of the
+                // pencil (0 .. Nax), as the reference's loop: a segment owns
+                // the interfaces at its cells' left, the last also Nax
+                T.nitmax = max(T.nitmax, nit);
+                if (nit < 0 && it - 5 >= skip && (it < last || s0 + len == Nax)) ++rare[1];
             }
             if constexpr (EARLY) deliver();
             else load(qn);
-            if (kk >= s0 + 3) {     // update cell k-3
+            if (it >= 6 && it - 6 >= skip) {   // update cell k-3
                 Flux Fprev;
                 Fprev.p = flux[0]; Fprev.r = flux[STREAM_BLOCK]; Fprev.u = flux[2 * STREAM_BLOCK];
                 Fprev.v = flux[3 * STREAM_BLOCK]; Fprev.w = flux[4 * STREAM_BLOCK];
@@ -818,8 +807,14 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
                              GRAV);
                 double val[5];
                 val[0] = pres; val[1] = rho; val[D::U] = u; val[D::V] = vv; val[D::W] = w;
-                const int ic = nb + kk - 3;
-                finish_cell<M, EXP>(B, E, A.gamma, q - 3 * s_ax, val, ixc, DIR == 2 ? ic : ibc, DIR == 2 ? ibc : ic, T);
+                settle_cell<M, EXP>(E, A.gamma, q - 3 * s_ax, val, T);
+                // the axis' own ghost images only from cells within 2 nb of its
+                // ends, asked of a scalar where the wave has one segment
+                const int ic = nb + s0 + it - 6, ic_wave = nb + s0_wave + it - 6;
+                const bool far = alone && ic_wave >= 2 * nb && ic_wave < Nax;
+                const int mask = far ? E.ghost_mask & ~(1 << (DIR - 1)) : E.ghost_mask;
+                store_cell(B.out, q - 3 * s_ax, val, ixc, DIR == 2 ? ic : ibc, DIR == 2 ? ibc : ic, mask, B.nx, B.ny,
+                           B.nz, nb);
             }
             flux[0] = F.p; flux[STREAM_BLOCK] = F.r; flux[2 * STREAM_BLOCK] = F.u;
             flux[3 * STREAM_BLOCK] = F.v; flux[4 * STREAM_BLOCK] = F.w;
@@ -830,6 +825,7 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
             for (int s = 0; s < NV; ++s) { d2[s] = d3[s]; iv2[s] = iv1[s]; }
             bits = (bits >> 1) | ((bk ? 1u : 0u) << 2);
             fRprev = fR;
+            q = qn;
         }
     }
 }
@@ -853,13 +849,12 @@ sweep_stream(BoxView B, Epilogue E, int seglen, int nseg)
     long s_ax, s_b;
     stream_geometry<DIR>(B, Nax, Nbb, s_ax, s_b);
     const unsigned wave = __builtin_amdgcn_readfirstlane((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    unsigned pen, seg;
-    const bool active = stream_item(wave, (unsigned)((B.nx - 2 * B.nb) * Nbb), pen, seg) && (int)seg < nseg;
+    const StreamItem I = stream_item(wave, threadIdx.x & 63u, (unsigned)((B.nx - 2 * B.nb) * Nbb), (unsigned)nseg);
     const AllScalars<R> A = wave_uniform(load_scalars<M, R>(B.prm, B.st));
     Tally T = tally0();
     double* const column = window + threadIdx.x;
     reset_rare<GRAV>(column);
-    stream_run<M, R, DIR, GRAV, COSMO, EXP>(B, A, E, pen, seg, seglen, active, T, column);
+    stream_run<M, R, DIR, GRAV, COSMO, EXP>(B, A, E, I.pen, (int)I.seg, seglen, I.active, T, column);
     take_rare<GRAV>(column, T);
     flush_counters_block(B.st, T, E.do_speed != 0);
 }
