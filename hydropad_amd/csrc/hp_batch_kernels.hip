@@ -95,7 +95,7 @@ template <class M, class R, int DIR, bool EXP>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, false, true>())))
 batch_stream(const BatchBox* __restrict__ boxes, const BatchPlan* __restrict__ plan, int key, int slot)
 {
-    __shared__ double window[stream_lds<false>() * STREAM_BLOCK];
+    __shared__ double window[stream_lds<false>() * 256];
     const BatchTable& T = plan->t[key];
     const int total = T.total;
     const int nwaves = (gridDim.x * blockDim.x) >> 6;
@@ -104,7 +104,7 @@ batch_stream(const BatchBox* __restrict__ boxes, const BatchPlan* __restrict__ p
     const int u0 = __builtin_amdgcn_readfirstlane((int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6));
     int cur = -1;
     Tally t = tally0();
-    double* const column = window + threadIdx.x;
+    double* const column = stream_column<false>(window);
     reset_rare<false>(column);
     for (int u = u0; u < total; u += nwaves) {
         const int i = __builtin_amdgcn_readfirstlane(table_find(T, u));

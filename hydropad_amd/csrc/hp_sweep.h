@@ -632,22 +632,28 @@ template <int DIR> __device__ __forceinline__ void stream_geometry(const BoxView
 // The window a thread slides along its segment lives in LDS, one column of
 // doubles per thread: a ring of the last four cells and the flux at the
 // interface behind.  Only the thread itself reads its column, so nothing
-// synchronises; consecutive lanes' columns are consecutive doubles.  Kept in
+// synchronises; consecutive lanes' columns are consecutive doubles, and a
+// wave's stand together, so a block takes LDS for the waves it has (160^3
+// FP64 noise in blocks of 64 threads: 701 us with room for 256, 373 us).  Kept in
 // registers the window took the gamma = 5/3 kernels to 229 of them and two
 // waves per SIMD, and the VALU was busy 71 % of the time (the x sweep's three
 // waves: 92 %); a third wave fits beside the window in LDS.  Measured, y sweep
 // in us with its segment length, before and after: 256^3 comoving FP64 1194 ->
 // 1042, mixed 1068 -> 907, 160^3 gamma 1.66666667 (one wave -> two) 656 -> 494;
 // the 512^3 tube is bound by HBM (10.7 GB, 3.8 TB/s) and stays (2782 -> 2850).
-constexpr int STREAM_BLOCK = 256;                      // threads per block at most
+constexpr int STREAM_COL = 64;                         // doubles from one of a column's to the next
 template <bool GRAV> constexpr int stream_window() { return 4 * (GRAV ? 6 : 5) + 5; }
-template <bool GRAV> constexpr int stream_lds() { return stream_window<GRAV>() + 1; }
+template <bool GRAV> constexpr int stream_lds() { return stream_window<GRAV>() + 1; }   // doubles per thread
+template <bool GRAV> __device__ __forceinline__ double* stream_column(double* window)
+{
+    return window + (threadIdx.x >> 6) * (stream_lds<GRAV>() * STREAM_COL) + (threadIdx.x & 63u);
+}
 
 // The tallies that hardly ever change, clamps and iterations that did not
 // converge, are the two words of the column's last double.
 template <bool GRAV> __device__ __forceinline__ int* rare_tallies(double* column)
 {
-    return (int*)(column + stream_window<GRAV>() * STREAM_BLOCK);
+    return (int*)(column + stream_window<GRAV>() * STREAM_COL);
 }
 
 template <bool GRAV> __device__ __forceinline__ void reset_rare(double* column)
@@ -687,8 +693,8 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
     const long base = (nb + ia) + (long)(nb + ib) * s_b + (long)nb * s_ax;   // interior cell 0 of the pencil
     const bool flat_always = A.mingradflat <= 0.0;
 
-    auto cell = [&](int it) { return column + (it & 3) * NV * STREAM_BLOCK; };   // cell loaded in iteration `it`
-    double* const flux = column + 4 * NV * STREAM_BLOCK;                          // flux at interface k-3
+    auto cell = [&](int it) { return column + (it & 3) * NV * STREAM_COL; };   // cell loaded in iteration `it`
+    double* const flux = column + 4 * NV * STREAM_COL;                          // flux at interface k-3
     int* const rare = rare_tallies<GRAV>(column);
     double w0r = 0.0;                        // rho of cell k-4
     R d1r = R(0), d2[NV];                    // slopes of cells k-3 (rho), k-2
@@ -735,9 +741,9 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
 #pragma unroll
                 for (int s = 0; s < NV; ++s) {
                     cur[s] = nxt[s];
-                    w3[s] = c1[s * STREAM_BLOCK];
-                    w2[s] = c2[s * STREAM_BLOCK];
-                    c0[s * STREAM_BLOCK] = cur[s];       // over cell k-4
+                    w3[s] = c1[s * STREAM_COL];
+                    w2[s] = c2[s * STREAM_COL];
+                    c0[s * STREAM_COL] = cur[s];       // over cell k-4
                 }
             }
             if constexpr (EARLY) load(qn);
@@ -760,13 +766,13 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
             for (int s = 0; s < NV; ++s) iv1[s] = M::iface(w2[s], w3[s], d2[s], d3[s]);
 
             const double* const w1 = cell(it - 3);                    // cell k-3
-            const double w1r = w1[VR * STREAM_BLOCK];
+            const double w1r = w1[VR * STREAM_COL];
             Face<double> fL = fRprev, fR = fRprev;
             if (it >= 4) {     // parabola and faces of cell k-2
                 int nclL = 0, nclR = 0;
                 const bool flat = flat_always || bits != 0u || bk;
                 M::template cell_faces<R, NV, GRAV, COSMO>(A, w2, iv2, iv1, w0r, w1r, w3[VR], cur[VR], d1r, d3[VR],
-                                                           w1[VP * STREAM_BLOCK], w3[VP], flat, fL, fR, nclL, nclR);
+                                                           w1[VP * STREAM_COL], w3[VP], flat, fL, fR, nclL, nclR);
                 // clamps once per interface of the pencil (0 .. Nax), as the
                 // reference's loop counts them: a segment takes those of its
                 // own cells, the pencil's ends one face beyond
@@ -786,7 +792,7 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
                 if (w1r > A.Rs.dmax * w2[VR]) {
                     const long q4 = q - 4 * s_ax;
                     peak_floor(A.Rs, F, at(B.in[1], q4 - s_ax), at(B.in[1], q4), w1r, w2[VR], at(B.in[D::U], q4),
-                               w1[VU * STREAM_BLOCK]);
+                               w1[VU * STREAM_COL]);
                 }
                 // iterations that did not converge once per interface of the
                 // pencil (0 .. Nax), as the reference's loop: a segment owns
@@ -798,12 +804,12 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
             else load(qn);
             if (it >= 6 && it - 6 >= skip) {   // update cell k-3
                 Flux Fprev;
-                Fprev.p = flux[0]; Fprev.r = flux[STREAM_BLOCK]; Fprev.u = flux[2 * STREAM_BLOCK];
-                Fprev.v = flux[3 * STREAM_BLOCK]; Fprev.w = flux[4 * STREAM_BLOCK];
-                double pres = w1[VP * STREAM_BLOCK], rho = w1r, u = w1[VU * STREAM_BLOCK];
-                double vv = w1[VV * STREAM_BLOCK], w = w1[VW * STREAM_BLOCK];
+                Fprev.p = flux[0]; Fprev.r = flux[STREAM_COL]; Fprev.u = flux[2 * STREAM_COL];
+                Fprev.v = flux[3 * STREAM_COL]; Fprev.w = flux[4 * STREAM_COL];
+                double pres = w1[VP * STREAM_COL], rho = w1r, u = w1[VU * STREAM_COL];
+                double vv = w1[VV * STREAM_COL], w = w1[VW * STREAM_COL];
                 const double etot = total_phys<DIR>(A.rgamma1, pres, rho, u, vv, w);
-                M::integrate(A.Is, Fprev, F, pres, rho, u, vv, w, etot, GRAV ? w1[(NV - 1) * STREAM_BLOCK] : 0.0,
+                M::integrate(A.Is, Fprev, F, pres, rho, u, vv, w, etot, GRAV ? w1[(NV - 1) * STREAM_COL] : 0.0,
                              GRAV);
                 double val[5];
                 val[0] = pres; val[1] = rho; val[D::U] = u; val[D::V] = vv; val[D::W] = w;
@@ -816,8 +822,8 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
                 store_cell(B.out, q - 3 * s_ax, val, ixc, DIR == 2 ? ic : ibc, DIR == 2 ? ibc : ic, mask, B.nx, B.ny,
                            B.nz, nb);
             }
-            flux[0] = F.p; flux[STREAM_BLOCK] = F.r; flux[2 * STREAM_BLOCK] = F.u;
-            flux[3 * STREAM_BLOCK] = F.v; flux[4 * STREAM_BLOCK] = F.w;
+            flux[0] = F.p; flux[STREAM_COL] = F.r; flux[2 * STREAM_COL] = F.u;
+            flux[3 * STREAM_COL] = F.v; flux[4 * STREAM_COL] = F.w;
             // slide the rest of the window
             w0r = w1r;
             d1r = d2[VR];
@@ -843,7 +849,7 @@ template <class M, class R, int DIR, bool GRAV, bool COSMO, bool EXP>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, GRAV, COSMO>())))
 sweep_stream(BoxView B, Epilogue E, int seglen, int nseg)
 {
-    __shared__ double window[stream_lds<GRAV>() * STREAM_BLOCK];
+    extern __shared__ double window[];                 // stream_lds doubles per thread
     if (EXP) load_factors(E);
     int Nax, Nbb;
     long s_ax, s_b;
@@ -852,7 +858,7 @@ sweep_stream(BoxView B, Epilogue E, int seglen, int nseg)
     const StreamItem I = stream_item(wave, threadIdx.x & 63u, (unsigned)((B.nx - 2 * B.nb) * Nbb), (unsigned)nseg);
     const AllScalars<R> A = wave_uniform(load_scalars<M, R>(B.prm, B.st));
     Tally T = tally0();
-    double* const column = window + threadIdx.x;
+    double* const column = stream_column<GRAV>(window);
     reset_rare<GRAV>(column);
     stream_run<M, R, DIR, GRAV, COSMO, EXP>(B, A, E, I.pen, (int)I.seg, seglen, I.active, T, column);
     take_rare<GRAV>(column, T);
@@ -893,11 +899,12 @@ static hipError_t launch_sweep_t(const BoxView& b, const SweepLaunch& L, hipStre
         const int nseg = (Nax + seglen - 1) / seglen;
         const long threads = stream_items((long)Nx * Nbb, nseg) * 64;
         const long grid = (threads + block - 1) / block;
+        const size_t lds = sizeof(double) * stream_lds<G>() * block;
         if (L.dir == 2)
-            hipLaunchKernelGGL((sweep_stream<M, R, 2, G, C, X>), dim3((unsigned)grid), dim3(block), 0, s, b, E,
+            hipLaunchKernelGGL((sweep_stream<M, R, 2, G, C, X>), dim3((unsigned)grid), dim3(block), lds, s, b, E,
                                seglen, nseg);
         else
-            hipLaunchKernelGGL((sweep_stream<M, R, 3, G, C, X>), dim3((unsigned)grid), dim3(block), 0, s, b, E,
+            hipLaunchKernelGGL((sweep_stream<M, R, 3, G, C, X>), dim3((unsigned)grid), dim3(block), lds, s, b, E,
                                seglen, nseg);
     }
     return hipGetLastError();

@@ -62,3 +62,16 @@ def test_throughput_sweeps_keep_two_waves(report):
     assert len(held) == 18, held
     for n in sod + held:
         assert batch.get(n, fast.get(n))["waves"] >= 2, (n, batch.get(n, fast.get(n)))
+
+
+FIELDS["LDS Size [bytes/block]"] = "lds"
+
+
+def test_stream_window_is_sized_by_the_block(report):
+    """The y/z sweeps' LDS window is asked for at launch, for the threads a
+    block has (hp_set_tiling's block): reserved for 256 threads whatever the
+    block, a 64-thread block's single wave held 53 KB and a CU three of them."""
+    sweeps = {n: r for n, r in report[0].items() if "sweep_stream" in n}
+    assert len(sweeps) == 48
+    for name, r in sweeps.items():
+        assert r["lds"] < 1024, (name, r)
