@@ -239,8 +239,8 @@ int tile_boxes(hp_batch* b)
             nchunks += ((long)(X.ny - 2 * X.nb) * (X.nz - 2 * X.nb) * X.nx + 57) / 58;
         }
     const int chunks = hp::x_chunks_per_wave(nchunks);
-    const int slots = 4 * std::min(persistent_grid(b), 3 * b->ncu);   // waves of a y/z sweep's grid
-    const int len = hp::stream_seglen(nax, slots, [&](int nseg) {
+    const int grid = std::min(persistent_grid(b), 3 * b->ncu), resident = (grid + b->ncu - 1) / b->ncu;
+    const int len = hp::stream_seglen(nax, (long)grid * hp::SIMDS / resident, resident, [&](int nseg) {
         const int l = (nax + nseg - 1) / nseg;
         long waves = 0;
         for (const hp::BatchBox& X : b->h_boxes)

@@ -92,7 +92,7 @@ __global__ void __launch_bounds__(256) batch_x(const BatchBox* __restrict__ boxe
 // gamma = 5/3, two else; held there the bodies fit without a spill, left to
 // itself the allocator takes a few registers more and a wave is lost.
 template <class M, class R, int DIR, bool EXP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, false, true>())))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves(M::G53, false))))
 batch_stream(const BatchBox* __restrict__ boxes, const BatchPlan* __restrict__ plan, int key, int slot)
 {
     __shared__ double window[stream_lds<false>() * 256];
@@ -140,8 +140,8 @@ static void launch_dir(const BatchBox* boxes, const BatchPlan* plan, int key, in
                        int ncu, hipStream_t s)
 {
     // blocks of four waves a CU holds: one for each wave of a SIMD
-    constexpr int X = sizeof(R) == 4 ? (M::G53 ? 4 : 3) : (M::G53 ? 3 : 2);
-    const int grid = std::min(most, ncu * (dir == 1 ? X : stream_waves<M, R, false, true>()));
+    constexpr int X = batch_x_waves(M::G53, sizeof(R) == 4), YZ = stream_waves(M::G53, false);
+    const int grid = std::min(most, ncu * (dir == 1 ? X : YZ));
     if (dir == 1) hipLaunchKernelGGL((batch_x<M, R, EXP>), dim3(grid), dim3(256), 0, s, boxes, plan, key, slot);
     else if (dir == 2)
         hipLaunchKernelGGL((batch_stream<M, R, 2, EXP>), dim3(grid), dim3(256), 0, s, boxes, plan, key, slot);

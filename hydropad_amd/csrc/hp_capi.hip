@@ -82,7 +82,7 @@ struct hp_ctx {
     hp::DevStatus* d_st;
     hp_params h_prm;
     hipStream_t stream;
-    int device;
+    int device, cus;
     int seglen;
     int xcpw;
     int block;
@@ -158,6 +158,7 @@ static int sweep(hp_ctx* c, int dir, int ghost_mask, int do_speed, bool expand =
     L.seglen = c->seglen;
     L.xcpw = c->xcpw;
     L.block = c->block;
+    L.cus = c->cus;
     L.precision = c->precision;
     L.grav = c->has_grav;
     L.cosmo = is_cosmo(c->h_prm);
@@ -251,7 +252,11 @@ int hp_create(int nx, int ny, int nz, int nbound, int precision, hp_ctx** out)
     c->ppos = c->pvel = nullptr;
     c->np = c->pcap = 0;
     c->dtat = 0.0;
-    if (hipGetDevice(&c->device) != hipSuccess) { delete c; return HP_E_HIP; }
+    if (hipGetDevice(&c->device) != hipSuccess ||
+        hipDeviceGetAttribute(&c->cus, hipDeviceAttributeMultiprocessorCount, c->device) != hipSuccess) {
+        delete c;
+        return HP_E_HIP;
+    }
     const size_t fbytes = c->ncell * sizeof(double);
     const size_t align = 256;
     const size_t fstride = (fbytes + align - 1) / align * align;

@@ -64,6 +64,7 @@ struct SweepLaunch {
     int seglen;       // streaming segment length for y/z sweeps (<= 0: stream_seglen)
     int xcpw;         // x sweep: chunks per wave (<= 0: x_chunks_per_wave)
     int block;        // threads per block
+    int cus;          // compute units of the device
     int precision;    // Precision
     bool grav, cosmo;
     bool g53;         // gamma == 5/3 with the derived scalars of hp_params_init: constant-folded kernels

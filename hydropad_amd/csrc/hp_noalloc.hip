@@ -27,10 +27,12 @@ static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 constexpr int MAX_DEVICES = 64;
 std::mutex g_mu;
 unsigned char* g_ptr[MAX_DEVICES];   // device address of `scratch` on each GPU, set once
+int g_cus[MAX_DEVICES];              // its compute units
 
 // Device address of this GPU's copy of `scratch` (the array's name is only a
-// host-side stand-in), looked up once per device with that device current.
-int scratch_of_current_device(unsigned char** out)
+// host-side stand-in) and its compute units, looked up once per device with
+// that device current.
+int scratch_of_current_device(unsigned char** out, int* cus)
 {
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess) return HP_E_HIP;
@@ -39,9 +41,12 @@ int scratch_of_current_device(unsigned char** out)
     if (!g_ptr[dev]) {
         void* p = nullptr;
         if (hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)) != hipSuccess || !p) return HP_E_HIP;
+        if (hipDeviceGetAttribute(&g_cus[dev], hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+            return HP_E_HIP;
         g_ptr[dev] = (unsigned char*)p;
     }
     *out = g_ptr[dev];
+    *cus = g_cus[dev];
     return HP_OK;
 }
 
@@ -78,7 +83,8 @@ extern "C" int hp_ppmsolver_noalloc(const hp_params* prm, const double* p, const
         for (int b = 0; b < 5; ++b)
             if ((const void*)in[a] == (const void*)out[b]) return HP_E_ARG;   // the sweep reads and writes apart
     unsigned char* base = nullptr;
-    int rc = scratch_of_current_device(&base);
+    int cus = 0;
+    int rc = scratch_of_current_device(&base, &cus);
     if (rc) return rc;
     hp::Params* d_prm = (hp::Params*)(base + PRM_OFF);
     hp::DevStatus* d_st = (hp::DevStatus*)(base + ST_OFF);
@@ -107,6 +113,7 @@ extern "C" int hp_ppmsolver_noalloc(const hp_params* prm, const double* p, const
     L.seglen = 0;
     L.xcpw = 0;
     L.block = 256;
+    L.cus = cus;
     L.precision = precision;
     L.grav = gforce != nullptr;
     L.cosmo = prm->dat != 0.0 || prm->at != 1.0 || prm->rat != 1.0;

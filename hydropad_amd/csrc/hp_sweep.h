@@ -836,17 +836,8 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
     }
 }
 
-// Waves per SIMD a y/z kernel is built for: what LDS holds of its window
-// (three blocks of 53 KB per CU, two of 61 KB with gravity), and the registers
-// left after it (at most 168 for three waves: the general-gamma and the
-// reference-order forms need 175 to 237).
-template <class M, class R, bool GRAV, bool COSMO> constexpr int stream_waves()
-{
-    return M::G53 && !GRAV && (COSMO || sizeof(R) == 4) ? 3 : 2;
-}
-
 template <class M, class R, int DIR, bool GRAV, bool COSMO, bool EXP>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves<M, R, GRAV, COSMO>())))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(stream_waves(M::G53, GRAV))))
 sweep_stream(BoxView B, Epilogue E, int seglen, int nseg)
 {
     extern __shared__ double window[];                 // stream_lds doubles per thread
@@ -892,8 +883,8 @@ static hipError_t launch_sweep_t(const BoxView& b, const SweepLaunch& L, hipStre
         int seglen = L.seglen;
         if (seglen <= 0) {
             const long npen = (long)Nx * Nbb;
-            const int slots = STREAM_SLOTS * stream_waves<M, R, G, C>();
-            seglen = stream_seglen(Nax, slots, [&](int nseg) { return stream_items(npen, nseg); });
+            seglen = stream_seglen(Nax, (long)L.cus * SIMDS, stream_waves(M::G53, G),
+                                   [&](int nseg) { return stream_items(npen, nseg); });
         }
         if (seglen > Nax) seglen = Nax;
         const int nseg = (Nax + seglen - 1) / seglen;

@@ -26,9 +26,18 @@ inline int x_chunks_per_wave(long nchunks)
     return n;
 }
 
-// Waves of a y/z sweep the chip holds at once, for each wave its SIMD holds:
-// 256 CUs x 4 SIMDs.
-constexpr int STREAM_SLOTS = 1024;
+// Waves per SIMD that a y/z kernel is built for and its launch fills: what LDS
+// holds of its window (three blocks of 53 KB per CU, two of 61 KB with
+// gravity), and the registers left after it (at most 168 for three waves: the
+// gamma = 5/3 forms need 129 to 168, the general-gamma and the reference-order
+// forms 175 to 237).
+constexpr int stream_waves(bool g53, bool grav) { return g53 && !grav ? 3 : 2; }
+
+// Waves per SIMD of the batch's x kernels, bound by their registers (four
+// waves: 128).
+constexpr int batch_x_waves(bool g53, bool mixed) { return (mixed ? 3 : 2) + (g53 ? 1 : 0); }
+
+constexpr int SIMDS = 4;   // per CU
 
 // Segments of a pencil that stand side by side in a wave: one where the box
 // has more than 32 pencils, else as many as fill its 64 lanes.  Measured, z
@@ -76,28 +85,36 @@ HP_TILING_FN StreamItem stream_item(unsigned wave, unsigned lane, unsigned npen,
 }
 
 // Segment length of a y/z sweep whose pencils are `nax` cells long and take
-// `waves(nseg)` waves when each is split into nseg segments.  A wave walks a
-// segment of len cells in len + 6 iterations, the first four of them cheap:
-// about len + 4 cells' time, and the waves run in rounds of `slots`.  The
-// split with the smallest rounds x (len + 4) is taken, at most 24 cells long:
-// short enough that the waves that got the most Newton iterations do not run
-// on alone, and that the rows two segments share are still in cache.  Measured, y sweep in us, by length (taken one in brackets):
-//   64^3 tube                 64: 155   16: 49   8: 33   [2]: 24
-//   96^3 comoving             48: 353   16: 133  7: 94   [5]: 96   4: 107
-//   128^3 comoving            64: 448   32: 245  16: 174 [11]: 167  10: 181
-//   192^3 comoving            64: 640   28: 503  24: 520 [20]: 475  18: 491
-//   256^3 comoving            64: 1053  32: 1010 24: 984 [22]: 1042 16: 1023
-//   512^3 tube                128: 3270 64: 3132 32: 2995 [20]: 2854 16: 2811
-// A length just past a full round (10 at 128^3, 24 at 192^3) is slower than
-// its neighbours.
-template <class Waves> inline int stream_seglen(int nax, int slots, Waves waves)
+// `waves(nseg)` waves when each is split into nseg segments, on `simds` SIMDs
+// that hold `resident` waves each.  A wave walks a segment of len cells in
+// len + 6 iterations, the first four of them cheap: about len + 4 cells' time.
+// The waves run in rounds of simds x resident; a round that puts m waves on a
+// SIMD takes 1 + 0.3 (m - 1) of one wave's time alone (96^3 comoving, us per
+// cell at one, two and three waves: 6.8, 8.8, 10.9).  The split with the
+// shortest time is taken, at most 24 cells long: the waves that got the most
+// Newton iterations must not run on alone, and the rows two segments share
+// should still be in cache.  Measured, y sweep in us, by length (taken one in
+// brackets; over 46 sweeps of 64^3 to 512^3 it is 1.1 % off the best length on
+// average, 5.9 % at most):
+//   64^3 tube        64: 152   16: 50   8: 33   4: 25   [2]: 23.8   1: 30
+//   96^3 comoving    48: 363   16: 137  [7]: 95.5  5: 98.3  4: 109
+//   96^3 tube        48: 115   16: 48   [7]: 35.5  5: 36.8  4: 42.7
+//   128^3 comoving   64: 463   32: 255  15: 171 [11]: 172  10: 187
+//   160^3 comoving   32: 353   [23]: 337  20: 392  13: 323  11: 324  7: 324
+//   192^3 comoving   64: 664   32: 591  24: 536 [20]: 494  16: 514  12: 501
+//   256^3 comoving   64: 1142  32: 1091 24: 1068 [22]: 1074 16: 1110 12: 1115
+//   512^3 tube       128: 3268 64: 3142 32: 3014 24: 2924 [19]: 2858 16: 2813
+// 160^3 and 192^3 show what the rounds leave out: one or two of them balance
+// the Newton work less well than three or four shorter ones (3 to 6 %).
+template <class Waves> inline int stream_seglen(int nax, long simds, int resident, Waves waves)
 {
     int best = nax;
     long cost = -1;
     for (int most = nax < 24 ? nax : 24; most >= 1; --most) {
         const int shares = (nax + most - 1) / most, len = (nax + shares - 1) / shares;   // even shares
-        const long rounds = (waves((nax + len - 1) / len) + slots - 1) / slots;
-        const long c = rounds * (len + 4);
+        const long n = (waves((nax + len - 1) / len) + simds - 1) / simds;   // waves per SIMD
+        const long part = n % resident;
+        const long c = (len + 4) * (n / resident * (7 + 3 * resident) + (part ? 7 + 3 * part : 0));
         if (cost < 0 || c < cost) { cost = c; best = len; }
     }
     return best;

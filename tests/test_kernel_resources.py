@@ -65,6 +65,7 @@ def test_throughput_sweeps_keep_two_waves(report):
 
 
 FIELDS["LDS Size [bytes/block]"] = "lds"
+LDS_PER_CU = 160 << 10
 
 
 def test_stream_window_is_sized_by_the_block(report):
@@ -75,3 +76,44 @@ def test_stream_window_is_sized_by_the_block(report):
     assert len(sweeps) == 48
     for name, r in sweeps.items():
         assert r["lds"] < 1024, (name, r)
+
+
+CLAIMS = """
+#include <cstdio>
+#include "hp_tiling.h"
+int main()
+{
+    for (int g53 = 0; g53 < 2; ++g53)
+        for (int x = 0; x < 2; ++x)
+            std::printf("%d %d %d %d\\n", g53, x, hp::stream_waves(g53, x), hp::batch_x_waves(g53, x));
+}
+"""
+
+
+def test_kernels_hold_the_waves_their_launches_fill(report, tmp_path):
+    """The segment length of a y/z sweep and the batch's grids are sized to the
+    waves per SIMD that hp_tiling.h states: each kernel holds exactly those, by
+    its registers and, for the y/z sweeps, by the LDS of its window (26
+    doubles a thread, 30 with gravity, in blocks of 256)."""
+    (tmp_path / "claims.cpp").write_text(CLAIMS)
+    exe = str(tmp_path / "claims")
+    subprocess.run(["g++", "-std=c++17", "-I", build.CSRC, str(tmp_path / "claims.cpp"), "-o", exe], check=True)
+    stream, batch_x = {}, {}
+    for line in subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split("\n")[:-1]:
+        g53, x, s, b = map(int, line.split())
+        stream[g53, x], batch_x[g53, x] = s, b
+    checked = 0
+    for rep in report:
+        for name, r in rep.items():
+            g53 = "FastMath53" in name
+            form = re.search(r"FastMath(?:53)?E([df])(?:Li[23]E)?Lb([01])E", name)
+            if "stream" in name:
+                grav = "sweep_stream" in name and form.group(2) == "1"
+                lds = max(r["lds"], (30 if grav else 26) * 8 * 256 + (r["lds"] if "sweep_stream" in name else 0))
+                assert min(r["waves"], LDS_PER_CU // lds) == stream[g53, grav], (name, r)
+            elif "batch_x" in name:
+                assert r["waves"] == batch_x[g53, form.group(1) == "f"], (name, r)
+            else:
+                continue
+            checked += 1
+    assert checked == 48 + 16 + 8

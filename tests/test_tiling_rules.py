@@ -19,10 +19,10 @@ void item(unsigned wave, unsigned lane, unsigned npen, unsigned nseg, int* out)
     const hp::StreamItem i = hp::stream_item(wave, lane, npen, nseg);
     out[0] = i.active; out[1] = (int)i.pen; out[2] = (int)i.seg;
 }
-int seglen(int nax, long npen, int slots, int* tried)
+int seglen(int nax, long npen, int simds, int* tried)
 {
     int n = 0;
-    const int len = hp::stream_seglen(nax, slots, [&](int nseg) { ++n; return hp::stream_items(npen, nseg); });
+    const int len = hp::stream_seglen(nax, simds, 3, [&](int nseg) { ++n; return hp::stream_items(npen, nseg); });
     *tried = n;
     return len;
 }
@@ -85,6 +85,6 @@ def test_threads_fit_a_grid(rules):
 def test_segment_length_takes_few_steps(rules, nax):
     tried = ctypes.c_int()
     for npen in (9, 64, 4096, 1 << 18):
-        n = rules.seglen(nax, npen, 3072, ctypes.byref(tried))
+        n = rules.seglen(nax, npen, 1024, ctypes.byref(tried))
         assert 1 <= n <= min(nax, 24), npen
         assert tried.value <= 24, npen
