@@ -223,35 +223,24 @@ int push_box(hp_batch* b, int id)
 }
 
 // Work units of every active box, before a step that follows a change of the
-// boxes or of the tuning.  What a tuning leaves open is one for the whole
-// batch, by the rules of the single-box sweeps (x_chunks_per_wave,
-// stream_seglen) on all boxes' chunks and waves, these against the waves of
-// the persistent grid.  Eight comoving boxes of 32^3 to 64^3, 40 steps with
+// boxes or of the tuning: what a tuning leaves open is one for the boxes of a
+// form (form_tiling).  Eight comoving boxes of 32^3 to 64^3, 40 steps with
 // their uploads and downloads: 57.5 ms with whole pencils, 30.1 ms with this
 // rule, 25 ms with the window in LDS.
 int tile_boxes(hp_batch* b)
 {
-    int nax = 1;
-    long nchunks = 0;
+    std::vector<hp::BatchShape> shapes;
     for (const hp::BatchBox& X : b->h_boxes)
-        if (X.active) {
-            nax = std::max(nax, std::max(X.ny, X.nz) - 2 * X.nb);
-            nchunks += ((long)(X.ny - 2 * X.nb) * (X.nz - 2 * X.nb) * X.nx + 57) / 58;
-        }
-    const int chunks = hp::x_chunks_per_wave(nchunks);
-    const int grid = std::min(persistent_grid(b), 3 * b->ncu), resident = (grid + b->ncu - 1) / b->ncu;
-    const int len = hp::stream_seglen(nax, (long)grid * hp::SIMDS / resident, resident, [&](int nseg) {
-        const int l = (nax + nseg - 1) / nseg;
-        long waves = 0;
-        for (const hp::BatchBox& X : b->h_boxes)
-            if (X.active) {
-                const long Nx = X.nx - 2 * X.nb, Ny = X.ny - 2 * X.nb, Nz = X.nz - 2 * X.nb;
-                waves += hp::stream_items(Nx * Ny, (int)((Nz + l - 1) / l));
-            }
-        return waves;
-    });
+        if (X.active)
+            shapes.push_back({X.nx - 2 * X.nb, X.ny - 2 * X.nb, X.nz - 2 * X.nb, X.g53 != 0, X.prec == hp::PREC_MIXED});
+    hp::FormTiling T[hp::BATCH_FORMS];
+    for (int f = 0; f < hp::BATCH_FORMS; ++f)
+        T[f] = hp::form_tiling(shapes.data(), (int)shapes.size(), f, persistent_grid(b), b->ncu);
     for (hp::BatchBox& X : b->h_boxes)
-        if (X.active) set_units(X, b->tune, chunks, len);
+        if (X.active) {
+            const hp::FormTiling& F = T[hp::batch_form(X.g53 != 0, X.prec == hp::PREC_MIXED)];
+            set_units(X, b->tune, F.chunks, F.len);
+        }
     if (b->nbox > 0)
         HPCHK(hipMemcpyAsync(b->d_boxes, b->h_boxes.data(), sizeof(hp::BatchBox) * b->nbox, hipMemcpyHostToDevice,
                              b->stream));

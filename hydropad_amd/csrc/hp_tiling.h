@@ -120,4 +120,49 @@ template <class Waves> inline int stream_seglen(int nax, long simds, int residen
     return best;
 }
 
+// A box of a batch: its interior and the kernels that sweep it.
+struct BatchShape {
+    int Nx, Ny, Nz;
+    bool g53, mixed;
+};
+constexpr int BATCH_FORMS = 4;
+HP_TILING_FN int batch_form(bool g53, bool mixed) { return 2 * mixed + g53; }
+
+// x chunks per unit and y/z segment length of the boxes of one form: a launch
+// holds those, so they are dealt out by the rules of the single-box sweeps on
+// their chunks and waves, the latter against a persistent grid of `blocks` of
+// four waves, at most three to a CU.  Measured, ms per step, all boxes dealt
+// out together and by form: 48^3 and two 64^3 in each of the four forms 1.39
+// -> 0.92, 48^3 to 96^3 in both precisions 0.87 -> 0.73.  Three to a CU stands
+// for the general-gamma kernels too, though they hold two: with two counted
+// the segments came out longer and no batch faster (48^3 to 96^3 0.54 -> 0.58).
+struct FormTiling {
+    int chunks, len;
+};
+inline FormTiling form_tiling(const BatchShape* boxes, int n, int form, int blocks, int ncu)
+{
+    const auto in_form = [&](const BatchShape& X) { return batch_form(X.g53, X.mixed) == form; };
+    int nax = 1;
+    long nchunks = 0;
+    for (int i = 0; i < n; ++i) {
+        const BatchShape& X = boxes[i];
+        if (!in_form(X)) continue;
+        nax = X.Ny > nax ? X.Ny : nax;
+        nax = X.Nz > nax ? X.Nz : nax;
+        nchunks += ((long)X.Ny * X.Nz * (X.Nx + 6) + 57) / 58;
+    }
+    const int grid = blocks < 3 * ncu ? blocks : 3 * ncu;
+    const int resident = (grid + ncu - 1) / ncu;
+    FormTiling T;
+    T.chunks = x_chunks_per_wave(nchunks);
+    T.len = stream_seglen(nax, (long)grid * SIMDS / resident, resident, [&](int nseg) {
+        const int l = (nax + nseg - 1) / nseg;
+        long waves = 0;
+        for (int i = 0; i < n; ++i)
+            if (in_form(boxes[i])) waves += stream_items((long)boxes[i].Nx * boxes[i].Ny, (boxes[i].Nz + l - 1) / l);
+        return waves;
+    });
+    return T;
+}
+
 }  // namespace hp

@@ -11,6 +11,7 @@ import pytest
 from hydropad_amd import build
 
 SRC = r"""
+#include <vector>
 #include "hp_tiling.h"
 extern "C" {
 long items(long npen, long nseg) { return hp::stream_items(npen, nseg); }
@@ -25,6 +26,13 @@ int seglen(int nax, long npen, int simds, int* tried)
     const int len = hp::stream_seglen(nax, simds, 3, [&](int nseg) { ++n; return hp::stream_items(npen, nseg); });
     *tried = n;
     return len;
+}
+void forms(const int* boxes, int n, int form, int blocks, int ncu, int* out)
+{
+    std::vector<hp::BatchShape> v;
+    for (int i = 0; i < n; ++i, boxes += 5) v.push_back({boxes[0], boxes[1], boxes[2], boxes[3] != 0, boxes[4] != 0});
+    const hp::FormTiling t = hp::form_tiling(v.data(), n, form, blocks, ncu);
+    out[0] = t.chunks; out[1] = t.len;
 }
 }
 """
@@ -88,3 +96,22 @@ def test_segment_length_takes_few_steps(rules, nax):
         n = rules.seglen(nax, npen, 1024, ctypes.byref(tried))
         assert 1 <= n <= min(nax, 24), npen
         assert tried.value <= 24, npen
+
+
+def test_each_form_of_a_batch_is_dealt_out_by_itself(rules):
+    """A launch of a batch holds the boxes of one form (precision and gamma =
+    5/3 or not), so the others do not lengthen its segments."""
+    def tiling(boxes, g53, mixed, blocks=1024):
+        flat = (ctypes.c_int * (5 * len(boxes)))(*[v for b in boxes for v in b])
+        out = (ctypes.c_int * 2)()
+        rules.forms(flat, len(boxes), 2 * mixed + g53, blocks, 256, out)
+        return tuple(out)
+
+    all_boxes = [(n, n, n, g53, mixed) for n in (32, 48, 64) for g53 in (0, 1) for mixed in (0, 1)]
+    for g53 in (0, 1):
+        for mixed in (0, 1):
+            alone = [b for b in all_boxes if b[3:] == (g53, mixed)]
+            assert tiling(all_boxes, g53, mixed) == tiling(alone, g53, mixed)
+    for n in (64, 96, 128, 160):
+        tried = ctypes.c_int()
+        assert tiling([(n, n, n, 1, 0)], 1, 0)[1] == rules.seglen(n, n * n, 1024, ctypes.byref(tried))
