@@ -221,7 +221,7 @@ def serve(requests, hbm_budget=64 << 30, max_boxes=64, use_graph=True, keep_fiel
         ptrs = (_P * (5 * nreq))()
         for i in keep_fields:
             n = requests[i]["n"] + 6
-            fields[i] = field_arrays((n, n, n))
+            fields[i] = {k: np.zeros((n, n, n), dtype=np.float64, order="F") for k in FIELDS}
             for j, k in enumerate(FIELDS):
                 ptrs[5 * i + j] = fields[i][k].ctypes.data
     check("hp_serve_run", L.hp_serve_run(arr, nreq, int(hbm_budget), int(max_boxes), 1 if use_graph else 0, ptrs,
