@@ -20,11 +20,11 @@ def noisy_box(shape_interior, seed, amp, vamp):
     return ic.periodic_fill({k: np.asfortranarray(v) for k, v in st.items()})
 
 
-def run(st, P, d, seglen, precision="fp64"):
+def run(st, P, d, seglen, precision="fp64", gforce=None):
     with hp.Box(st["p"].shape, precision) as box:
         box.set_params(to_hp_params(P, hp.HpParams))
         box.set_tiling(0, seglen, 0)
-        box.upload(copy_state(st))
+        box.upload(copy_state(st), gforce)
         box.reset_counters()
         box.ppmsolver(d)
         return box.counters(), box.download()
@@ -55,3 +55,43 @@ def test_narrow_boxes(oracle, across, n):
                     assert np.array_equal(out[k], base[0][k]), (shape, d, wild, seglen, k)
                     if not wild:
                         assert rel_l1(out[k], ref[k]) <= 1e-12, (shape, d, seglen, k, rel_l1(out[k], ref[k]))
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed", "fp64_exact"])
+@pytest.mark.parametrize("gravity", [False, True], ids=["free", "gravity"])
+@pytest.mark.parametrize("comoving", [False, True], ids=["static", "comoving"])
+@pytest.mark.parametrize("gamma", [5.0 / 3.0, 1.66666667], ids=["5/3", "namelist"])
+def test_segments_of_every_form(oracle, precision, gravity, comoving, gamma):
+    """Pencils of 61 and 53 cells, whole (the window goes round 16 times) and
+    in segments of 1, 7 and the launch's own length: on a mild box the oracle's
+    values (relative L1 1e-12, mixed 2e-6) and the same bits, on a wild one
+    (Courant number 4) the same bits and the oracle's count of clamped states,
+    which there are, and, in the reference's order, of Newton iterations."""
+    shape = (11, 61, 53)
+    rng = np.random.default_rng(17)
+    g = np.asfortranarray(0.05 * (rng.random((3,) + tuple(n + 2 * NB for n in shape)) - 0.5)) if gravity else None
+    for wild in (False, True):
+        st = noisy_box(shape, 23, *((3.0, 2.0) if wild else (0.4, 0.4)))
+        P = oracle.params(gamma=gamma, ngrid=61)
+        oracle.timedet(P, oracle.speed(P, st), 4.0 if wild else 0.4, 1e30, 0.0)
+        if comoving:
+            P.at, P.dat, P.rat, P.rdtath = 0.8, 0.5, 1.25, P.dt / 0.81
+        for d in (2, 3):
+            ref, cnt = copy_state(st), OracleCounters()
+            oracle.ppmsolver(P, ref, d, gforce=g, counters=cnt)
+            assert cnt.neg_state_clamps > 0 or not wild
+            base = None
+            for seglen in (4096, 0, 1, 7):
+                c, out = run(st, P, d, seglen, precision, g)
+                base = base or (c, out)
+                if precision != "mixed":
+                    assert c.neg_state_clamps == cnt.neg_state_clamps, (d, wild, seglen)
+                if precision == "fp64_exact":
+                    assert c.newton_iters_max == cnt.newton_iters_max, (d, wild, seglen)
+                for name in ("neg_state_clamps", "newton_iters_max", "newton_nonconv"):
+                    assert getattr(c, name) == getattr(base[0], name), (d, wild, seglen, name)
+                for k in FIELDS:
+                    assert np.array_equal(out[k], base[1][k]), (d, wild, seglen, k)
+                    if not wild:
+                        assert rel_l1(out[k], ref[k]) <= (2e-6 if precision == "mixed" else 1e-12), \
+                            (d, seglen, k, rel_l1(out[k], ref[k]))
