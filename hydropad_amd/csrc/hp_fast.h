@@ -949,11 +949,13 @@ __device__ __forceinline__ Flux riemann_solve(const RScal& Rs, const Face<double
 // Dual-energy selection of integrate.F90:196-216 with the ratio tests
 // e_aux/E >= eta cross-multiplied when E > 0 (the reference's division
 // otherwise).
+template <bool X>
 __device__ __forceinline__ void dual_energy_d(const IScal& S, double etotnew, double rhonew, double vxnew,
                                               double vynew, double vznew, double eint, double pres,
                                               double& eintnew, double& pnew)
 {
-    const double vvv = vxnew * vxnew + vynew * vynew + vznew * vznew;
+    const double vvv = X ? vxnew * vxnew + vynew * vynew + vznew * vznew
+                         : fma(vznew, vznew, fma(vxnew, vxnew, vynew * vynew));
     const double eeaux = etotnew - 0.50 * rhonew * vvv;
     bool ge2, ge1;
     if (etotnew > 0.0) {
@@ -969,6 +971,7 @@ __device__ __forceinline__ void dual_energy_d(const IScal& S, double etotnew, do
     if (eintnew <= 0.0) { eintnew = eint; pnew = pres; }
 }
 
+template <bool X>
 __device__ __forceinline__ void integrate_cell(const IScal& S, const Flux& F1, const Flux& F2, double& pres,
                                                double& rho, double& vx, double& vy, double& vz, double etot,
                                                double ghalf, bool grav)
@@ -981,20 +984,29 @@ __device__ __forceinline__ void integrate_cell(const IScal& S, const Flux& F1, c
     double px = vx * rho + lam * ((m1 * F1.u + F1.p) - (m2 * F2.u + F2.p));
     if (grav) px += S.rdtath * ((rho + rhonew) * ghalf * 0.5);
     const double vxnew = px * rrn;
-    // which product is rounded is written out: left to the compiler, the x and
-    // the y/z sweeps round the transverse momenta differently
+    // Which product is rounded is written out for the transverse momenta and,
+    // in the y/z sweeps, for the enthalpies and the kinetic energy
+    // (dual_energy_d): left to the compiler, a y/z interface's energy flux was
+    // rounded one way for the cell on its left and another for the cell on its
+    // right once the flux behind came from LDS, an ulp of the pressure.  Gas at
+    // rest under gravity amplifies such an ulp to 1e-8 in pressure over eight
+    // steps of a planar tube.  The x sweeps keep the compiler's choice, which
+    // rounds as it always did.
     auto momentum = [&](double r, double v, double d) { return fma(r, v, lam * d); };
     const double vynew = momentum(rho, vy, F1.v * m1 - F2.v * m2) * rrn;
     const double vznew = momentum(rho, vz, F1.w * m1 - F2.w * m2) * rrn;
-    const double e1 = (gamma * F1.p * rgamma1 + 0.5 * F1.r * (F1.u * F1.u + F1.v * F1.v + F1.w * F1.w)) * F1.u;
-    const double e2 = (gamma * F2.p * rgamma1 + 0.5 * F2.r * (F2.u * F2.u + F2.v * F2.v + F2.w * F2.w)) * F2.u;
+    auto enthalpy = [&](const Flux& F) {
+        if (X) return gamma * F.p * rgamma1 + 0.5 * F.r * (F.u * F.u + F.v * F.v + F.w * F.w);
+        return fma(0.5 * F.r, fma(F.w, F.w, fma(F.v, F.v, F.u * F.u)), gamma * F.p * rgamma1);
+    };
+    const double e1 = enthalpy(F1) * F1.u, e2 = enthalpy(F2) * F2.u;
     double etotnew = etot + lam * (e1 - e2);
     if (grav) etotnew += S.rdtath * ((rho * vx + rhonew * vxnew) * ghalf * 0.5);
     const double pmean = (F1.p + F2.p) * 0.5;
     double eintnew = eint + lam * (pmean * (F1.u - F2.u) + (F1.p * F1.u - F2.p * F2.u) * rgamma1);
     if (eintnew < 0.0) eintnew = eint;
     double pnew;
-    dual_energy_d(S, etotnew, rhonew, vxnew, vynew, vznew, eint, pres, eintnew, pnew);
+    dual_energy_d<X>(S, etotnew, rhonew, vxnew, vynew, vznew, eint, pres, eintnew, pnew);
     if (rhonew <= 0.0) rhonew = rho;
     pres = pnew;
     rho = rhonew;

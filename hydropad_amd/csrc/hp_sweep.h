@@ -56,6 +56,7 @@ struct ExactMath {
     {
         return riemann_solve(Rs, L, Rt, nit);
     }
+    template <bool X>
     static __device__ __forceinline__ void integrate(const IScal& S, const Flux& F1, const Flux& F2, double& p,
                                                      double& rho, double& u, double& v, double& w, double etot,
                                                      double g, bool grav)
@@ -89,11 +90,12 @@ struct FastMath {
     {
         return fm::riemann_solve<R>(Rs, L, Rt, nit);
     }
+    template <bool X>
     static __device__ __forceinline__ void integrate(const IScal& S, const Flux& F1, const Flux& F2, double& p,
                                                      double& rho, double& u, double& v, double& w, double etot,
                                                      double g, bool grav)
     {
-        fm::integrate_cell(S, F1, F2, p, rho, u, v, w, etot, g, grav);
+        fm::integrate_cell<X>(S, F1, F2, p, rho, u, v, w, etot, g, grav);
     }
     // the CFL sound speed keeps speed.F90's IEEE sqrt(gamma*p/rho), so the
     // fused maximum equals hp_speed's bit for bit and every path gets the same dt
@@ -594,7 +596,7 @@ __device__ __forceinline__ void x_run(const BoxView& B, const AllScalars<R>& A, 
             }
             double pres = cd[VP], rho = cd[VR], u = cd[VU], vv = cd[VV], w = cd[VW];
             const double etot = total_phys<1>(A.rgamma1, pres, rho, u, vv, w);
-            M::integrate(A.Is, F, F2, pres, rho, u, vv, w, etot, GRAV ? cd[NV - 1] : 0.0, GRAV);
+            M::template integrate<true>(A.Is, F, F2, pres, rho, u, vv, w, etot, GRAV ? cd[NV - 1] : 0.0, GRAV);
             double val[5];
             val[0] = pres; val[1] = rho; val[D::U] = u; val[D::V] = vv; val[D::W] = w;
             finish_cell<M, EXP>(B, E, A.gamma, q, val, i, j, k, T);
@@ -809,7 +811,7 @@ __device__ __forceinline__ void stream_run(const BoxView& B, const AllScalars<R>
                 double pres = w1[VP * STREAM_COL], rho = w1r, u = w1[VU * STREAM_COL];
                 double vv = w1[VV * STREAM_COL], w = w1[VW * STREAM_COL];
                 const double etot = total_phys<DIR>(A.rgamma1, pres, rho, u, vv, w);
-                M::integrate(A.Is, Fprev, F, pres, rho, u, vv, w, etot, GRAV ? w1[(NV - 1) * STREAM_COL] : 0.0,
+                M::template integrate<false>(A.Is, Fprev, F, pres, rho, u, vv, w, etot, GRAV ? w1[(NV - 1) * STREAM_COL] : 0.0,
                              GRAV);
                 double val[5];
                 val[0] = pres; val[1] = rho; val[D::U] = u; val[D::V] = vv; val[D::W] = w;
