@@ -385,13 +385,21 @@ __device__ __forceinline__ Face<double> trace_face_d(const SweepScalars<R>& S, c
     // those terms a face of gas at rest or moving the other way is its traced
     // state as it stands: each cell then corrects at most one face, and a
     // wave of gas at rest none (512^3 tube, 3 steps: 45.1 -> 41.6 ms; the
-    // comoving sweeps, which keep the expansion terms, unchanged).
+    // comoving sweeps, which keep the expansion terms, unchanged).  A face
+    // whose sound speed or velocity is no normal number (p rho underflows, an
+    // infinity or a NaN comes in) is corrected by every term, so that it ends
+    // as it does there: its cells keep their state instead of turning NaN.
     const bool away = RIGHT ? (u0 > 0.0) : (u0 < 0.0);
+    bool whole = pneg;
+    if constexpr (!GRAV && !COSMO) {
+        constexpr int POSITIVE_NORMAL = 1 << 8;
+        whole = whole || !__builtin_amdgcn_class(fma((double)ut, 0.0, ptl * rtl), POSITIVE_NORMAL);
+    }
     Face<double> f;
     f.p = ptl;
     f.r = rtl;
     R du = ut;
-    if (GRAV || COSMO || away || pneg) {
+    if (GRAV || COSMO || away || whole) {
         // the Lagrangian sound speed and its inverse (order2interp.F90:192-193):
         // in FP64 both from one rsq; in FP32 the hardware root and reciprocal
         R ct, rct;
@@ -407,7 +415,7 @@ __device__ __forceinline__ Face<double> trace_face_d(const SweepScalars<R>& S, c
         const R xo = RIGHT ? x3 : x1, xi = RIGHT ? x1 : x3;
         R bo = R(0), bi = R(0), b0 = R(0);
         if (RIGHT ? (up > 0.0) : (um < 0.0)) {
-            if (pneg) {
+            if (whole) {
                 const R pc = tr(q[VP], xo);
                 bo = beta_d<R, GRAV, COSMO>(S, rct, ut, ut, pt, pc, ap + pc, au + ut, gravity(xo), R(so));
             } else if (GRAV || COSMO) {
