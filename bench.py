@@ -110,17 +110,20 @@ def roofline_of(r, N, prec):
            "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
            "alg_bytes_per_launch": alg_bytes, "avg_ms_per_launch": per_dir}
     # the issue floor: the dominant kernel's VALU instructions per launch (SQ
-    # counters of the same workload, profiles/valu.json) at one wave64
-    # instruction per 4 cycles on each of 1024 SIMDs at 2.4 GHz, against the
-    # launch time measured here
+    # counters of the same workload over the same number of steps,
+    # profiles/valu.json) at one wave64 instruction per 4 cycles on each of
+    # 1024 SIMDs at 2.4 GHz, against the launch time measured here; none where
+    # that number of steps was not counted, as the count grows with the tube
     if os.path.exists(VALU_FILE):
         try:
             v = json.load(open(VALU_FILE)).get(f"{names[dom]}@{N}@{prec}")
-            if v:
-                out["valu_issue"] = {"insts_per_launch": v["valu_insts_per_launch"],
-                                     "insts_per_64_cells": v["valu_insts_per_64_cells"],
-                                     "issue_bound_ms": v["issue_bound_ms"],
-                                     "frac": round(v["issue_bound_ms"] / avg_ms, 4)}
+            insts = v["by_launches"].get(str(r["launches"][dom])) if v else None
+            if insts:
+                bound_ms = insts * 4 / (1024 * 2.4e9) * 1e3
+                out["valu_issue"] = {"insts_per_launch": insts,
+                                     "insts_per_64_cells": round(insts / (N ** 3 / 64.0), 1),
+                                     "issue_bound_ms": round(bound_ms, 4),
+                                     "frac": round(bound_ms / avg_ms, 4)}
         except (ValueError, KeyError):
             pass
     return out

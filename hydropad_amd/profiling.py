@@ -122,6 +122,7 @@ def traffic_entries(fetch_db, write_db, size, precision, copy_bytes):
 # cycles (16 lanes per cycle, the FP64 and unpacked-FP32 rate) at the 2.4 GHz
 # peak engine clock
 SIMDS, VALU_CYCLES, CLOCK_HZ = 1024, 4, 2.4e9
+VALU_LAUNCHES = (1, 2, 3, 5, 10, 20, 30, 50, 100, 200, 300)
 
 
 def valu_entries(sq_db, size, precision):
@@ -129,19 +130,24 @@ def valu_entries(sq_db, size, precision):
     run: SQ_INSTS_VALU (wave instructions, averaged over every dispatch of
     the kernel) and the time the chip needs just to issue them,
     insts x 4 cycles / (1024 SIMDs x 2.4 GHz) -- the floor set by instruction
-    count alone, whatever the memory traffic."""
+    count alone, whatever the memory traffic.  The count of an x sweep doubles
+    as the tube develops, so `by_launches` gives the average over the first n
+    dispatches too: a run of n steps is held against those."""
     db = sqlite3.connect(sq_db)
     vals = collections.defaultdict(lambda: collections.defaultdict(list))
-    for name, cn, v in db.execute("select kernel_name, counter_name, value from counters_collection"):
+    for name, cn, v in db.execute("select kernel_name, counter_name, value from counters_collection "
+                                  "order by dispatch_id"):
         vals[name.split("(")[0]][cn].append(v)
     out = {}
     for k, d in vals.items():
         if "sweep" not in k or "SQ_INSTS_VALU" not in d:
             continue
         short = "sweep_lane_x" if "lane_x" in k else ("sweep_stream<y>" if ", 2," in k else "sweep_stream<z>")
-        insts = float(np.mean(d["SQ_INSTS_VALU"]))
+        seq = d["SQ_INSTS_VALU"]
+        insts = float(np.mean(seq))
         out[f"{short}@{size}@{precision}"] = {
-            "valu_insts_per_launch": round(insts), "dispatches": len(d["SQ_INSTS_VALU"]),
+            "valu_insts_per_launch": round(insts), "dispatches": len(seq),
+            "by_launches": {str(n): round(float(np.mean(seq[:n]))) for n in VALU_LAUNCHES if n <= len(seq)},
             "valu_insts_per_64_cells": round(insts / (size ** 3 / 64.0), 1),
             "issue_bound_ms": round(insts * VALU_CYCLES / (SIMDS * CLOCK_HZ) * 1e3, 4), "kernel": k}
     return out

@@ -47,3 +47,15 @@ def test_roofline_record_from_committed_profiles():
         assert abs(v["issue_bound_ms"] - v["insts_per_launch"] * 4 / (1024 * 2.4e9) * 1e3) < 1e-3
         assert abs(v["frac"] - v["issue_bound_ms"] / 8.0) < 1e-3
         assert 0.5 < v["frac"] <= 1.0
+
+
+def test_issue_floor_is_of_the_steps_timed():
+    """The x sweep's instruction count doubles as the tube develops, so a run of
+    20 steps is held against the first 20 launches' count, and a number of
+    steps that was not counted gets no issue figure."""
+    import bench
+    full, short, other = (bench.roofline_of({"ms": [n * 8.0, n * 3.5, n * 3.4], "launches": [n] * 3}, 512, "fp64")
+                          for n in (300, 20, 7))
+    assert short["valu_issue"]["insts_per_launch"] < 0.75 * full["valu_issue"]["insts_per_launch"]
+    assert abs(short["valu_issue"]["frac"] - short["valu_issue"]["insts_per_launch"] * 4 / (1024 * 2.4e9) / 8e-3) < 1e-3
+    assert "valu_issue" not in other
