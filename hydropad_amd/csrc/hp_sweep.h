@@ -642,7 +642,7 @@ template <int DIR> __device__ __forceinline__ void stream_geometry(const BoxView
 // waves: 92 %); a third wave fits beside the window in LDS.  Measured, y sweep
 // in us with its segment length, before and after: 256^3 comoving FP64 1194 ->
 // 1042, mixed 1068 -> 907, 160^3 gamma 1.66666667 (one wave -> two) 656 -> 494;
-// the 512^3 tube is bound by HBM (10.7 GB, 3.8 TB/s) and stays (2782 -> 2850).
+// the 512^3 tube is bound by HBM (13.3 GB, 4.7 TB/s) and stays (2782 -> 2850).
 constexpr int STREAM_COL = 64;                         // doubles from one of a column's to the next
 template <bool GRAV> constexpr int stream_window() { return 4 * (GRAV ? 6 : 5) + 5; }
 template <bool GRAV> constexpr int stream_lds() { return stream_window<GRAV>() + 1; }   // doubles per thread
