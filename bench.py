@@ -109,11 +109,13 @@ def roofline_of(r, N, prec):
     out = {"bound": "hbm", "kernel": names[dom], "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
            "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": traffic,
            "alg_bytes_per_launch": alg_bytes, "avg_ms_per_launch": per_dir}
-    # the issue floor: the dominant kernel's VALU instructions per launch (SQ
-    # counters of the same workload over the same number of steps,
-    # profiles/valu.json) at one wave64 instruction per 4 cycles on each of
-    # 1024 SIMDs at 2.4 GHz, against the launch time measured here; none where
-    # that number of steps was not counted, as the count grows with the tube
+    # VALU issue: the dominant kernel's instructions per launch (SQ counters of
+    # the same workload over the same number of steps, profiles/valu.json) at
+    # the nominal 4 cycles of a wave64 FP64 instruction on each of 1024 SIMDs
+    # at 2.4 GHz, against the launch time measured here; none where that number
+    # of steps was not counted, as the count grows with the tube.  32-bit
+    # instructions of two waves issue in half that, so the mixed form's
+    # fraction can pass 1
     if os.path.exists(VALU_FILE):
         try:
             v = json.load(open(VALU_FILE)).get(f"{names[dom]}@{N}@{prec}")

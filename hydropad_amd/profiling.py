@@ -118,9 +118,12 @@ def traffic_entries(fetch_db, write_db, size, precision, copy_bytes):
     return out
 
 
-# MI355X: 256 CUs x 4 SIMDs; a wave64 VALU instruction occupies its SIMD for 4
-# cycles (16 lanes per cycle, the FP64 and unpacked-FP32 rate) at the 2.4 GHz
-# peak engine clock
+# MI355X: 256 CUs x 4 SIMDs; nominally a wave64 FP64 instruction occupies its
+# SIMD for 4 cycles (16 lanes per cycle) at the 2.4 GHz peak engine clock.  A
+# loop of independent instructions, four waves per SIMD, measured in cycles of
+# 2.4 GHz: fma_f64 5.0, mul_f64 4.7, add_f64 4.4, cmp_f64 and mov_b64 4.3,
+# conversions 4.4, rcp_f64 16.4, rcp_f32 8.3; add_u32, mul_f32 and mov_b32
+# 2.3 to 2.6 (of two waves at once; alone 5)
 SIMDS, VALU_CYCLES, CLOCK_HZ = 1024, 4, 2.4e9
 VALU_LAUNCHES = (1, 2, 3, 5, 10, 20, 30, 50, 100, 200, 300)
 
@@ -129,8 +132,9 @@ def valu_entries(sq_db, size, precision):
     """VALU issue figures per launch of each sweep kernel from one SQ counter
     run: SQ_INSTS_VALU (wave instructions, averaged over every dispatch of
     the kernel) and the time the chip needs just to issue them,
-    insts x 4 cycles / (1024 SIMDs x 2.4 GHz) -- the floor set by instruction
-    count alone, whatever the memory traffic.  The count of an x sweep doubles
+    insts x 4 cycles / (1024 SIMDs x 2.4 GHz), at the nominal rate of FP64
+    instructions: a yardstick, as reciprocals take four times as long and
+    32-bit instructions half.  The count of an x sweep doubles
     as the tube develops, so `by_launches` gives the average over the first n
     dispatches too: a run of n steps is held against those."""
     db = sqlite3.connect(sq_db)
